@@ -4,6 +4,8 @@
 #ifndef CUDALM_W4A16_DEVICE_H
 #define CUDALM_W4A16_DEVICE_H
 
+#include <type_traits>
+
 #include "hip_common.h"
 
 namespace cudalm_hip {
@@ -80,6 +82,85 @@ __device__ __forceinline__ f32x4_t group_offset(const u32x4_t (&xa)[4]) {
   return c;
 }
 
+// Activation / output element type of a kernel instance. Both encode a
+// weight nibble as an exact value c + q/kUnit in the activation's 16-bit
+// format (the nibble in mantissa bits 3..6), cancel c with an MFMA against
+// -c, and scale the accumulated sum by kUnit in the epilogue.
+struct ActBf16 {
+  static constexpr uint32_t kNegOffsetPair = 0xBFC0BFC0u;  // -1.5, -1.5
+  static constexpr float kUnit = 16.0f;  // weight element = 1.5 + q / kUnit
+  template <bool ROT>
+  __device__ static u32x4_t decode(uint32_t w) { return decode_nibbles<ROT>(w); }
+  __device__ static f32x4_t mma(u32x4_t a, u32x4_t b, f32x4_t c) { return mfma16(a, b, c); }
+  __device__ static uint32_t round(float f) { return f32_to_bf16_rne(f); }
+  // two roundings in one dword (lo in bits 0..15): one v_cvt_pk_bf16_f32
+  __device__ static uint32_t round2(float lo, float hi) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2_t{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
+  }
+  __device__ static float widen(uint32_t h) { return bf16_lo(h); }
+};
+
+// fp16: 1.0 = 0x3C00 with 10 mantissa bits, so q/16 sits at bit 6 and the
+// biased nibble (q + 8 = nibble ^ 8) goes to bits 6..9: 0x3C00 | 0x0200 is
+// 1.5, and the element is exactly 1.5 + q/16, the bf16 element's value. One
+// shift (one rotation from the prepacked form, which is the file dword
+// rotated left by 3) and one v_bitop3 per pair: 8 VALU ops per dword.
+// Keeping the bias at 1.5 (not 1.0625 + q/128 with the nibble at bits
+// 3..6, one op less) keeps the fp32 cancellation of the offset chain as
+// small as in bf16: the reference fixtures then stay within 0.5 fp16 ulp.
+struct ActF16 {
+  static constexpr uint32_t kNegOffsetPair = 0xBE00BE00u;  // -1.5, -1.5
+  static constexpr float kUnit = 16.0f;  // weight element = 1.5 + q / kUnit
+  template <bool ROT>
+  __device__ static u32x4_t decode(uint32_t w) {
+    u32x4_t a;
+    if constexpr (ROT) {
+      a[0] = (rotr(w, 29) & 0x03C003C0u) ^ 0x3E003E00u;
+      a[1] = (rotr(w, 1) & 0x03C003C0u) ^ 0x3E003E00u;
+      a[2] = (rotr(w, 5) & 0x03C003C0u) ^ 0x3E003E00u;
+      a[3] = (rotr(w, 9) & 0x03C003C0u) ^ 0x3E003E00u;
+    } else {
+      a[0] = ((w << 6) & 0x03C003C0u) ^ 0x3E003E00u;
+      a[1] = ((w << 2) & 0x03C003C0u) ^ 0x3E003E00u;
+      a[2] = ((w >> 2) & 0x03C003C0u) ^ 0x3E003E00u;
+      a[3] = ((w >> 6) & 0x03C003C0u) ^ 0x3E003E00u;
+    }
+    return a;
+  }
+  __device__ static f32x4_t mma(u32x4_t a, u32x4_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
+  // round to nearest even (v_cvt_f16_f32 under the default rounding mode)
+  __device__ static uint32_t round(float f) {
+    return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
+  }
+  __device__ static uint32_t round2(float lo, float hi) { return round(lo) | round(hi) << 16; }
+  __device__ static float widen(uint32_t h) { return half_bits_to_f32(h & 0xFFFFu); }
+};
+
+// An activation trait bound to a weight layout: decode() reads file dwords
+// (PACKED false) or prepacked, rotated dwords (PACKED true).
+template <class Act, bool PACKED>
+struct Layout : Act {
+  __device__ static u32x4_t decode(uint32_t w) { return Act::template decode<PACKED>(w); }
+};
+
+// -1.5 * (sum over the group of this lane-set's activation rows) in the
+// activation type Act.
+template <class Act>
+__device__ __forceinline__ f32x4_t group_offset_t(const u32x4_t (&xa)[4]) {
+  const u32x4_t neg = {Act::kNegOffsetPair, Act::kNegOffsetPair, Act::kNegOffsetPair,
+                       Act::kNegOffsetPair};
+  const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t c = Act::mma(xa[0], neg, zero);
+  c = Act::mma(xa[1], neg, c);
+  c = Act::mma(xa[2], neg, c);
+  c = Act::mma(xa[3], neg, c);
+  return c;
+}
+
 // The reference's own loop for one output (tests/cuda/test_int4_gemv_bf16.cpp:
 // 54-69; the fp16 twin, tests/cuda/test_int4_gemv.cpp:49-63): fp32, k
 // ascending, each term (q * f32(s)) * f32(x). The kernels call it only for
@@ -126,6 +207,48 @@ __device__ __forceinline__ float w4a16_ref_dot(const uint8_t* W, const uint16_t*
   return acc;
 }
 
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// D = A (32 rows x 16 k) * B (16 k x 32 cols) + C in the activation type,
+// fp32 accumulate.
+template <class Act>
+__device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
+  if constexpr (std::is_same<Act, ActF16>::value)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// LDS layout of staged activations. A row holds K/8 16-byte blocks plus
+// kXPad pad blocks, so rows start 2 blocks (mod 16) apart, and inside each
+// 128-column group the block of lane quarter a, step d (logical block
+// 4a + d, columns 32a + 8d ..) sits at slot 4d + a. One ds_read_b128 step
+// of a wave then reads 4 adjacent blocks from each of 16 rows: measured
+// conflict-free on gfx950 (4 LDS cycles per instruction), where unswizzled
+// rows 1 block (mod 16) apart spend half their cycles in bank conflicts.
+constexpr int kXPad = 2;
+__host__ __device__ constexpr int x_pitch(int kcl) { return (kcl >> 3) + kXPad; }
+__device__ __forceinline__ int x_slot(int c) { return (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3); }
+
+__device__ __forceinline__ void load_group_x(u32x4_t (&xa)[4], const u32x4_t* xgroup, int a) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) xa[d] = xgroup[4 * d + a];
+}
+
+// The output of one accumulator: kUnit * total, or, when that is NaN, the
+// reference loop's sum for the output (w4a16_ref_dot: infinite and NaN
+// activations and overflow keep the reference's semantics).
+template <class Act, bool PACKED>
+__device__ __forceinline__ float out_value(float total, const uint8_t* w, const uint16_t* s, int K,
+                                           int n, const uint16_t* xrow) {
+  const float v = Act::kUnit * total;
+  if (__builtin_expect(v != v, 0))
+    return w4a16_ref_dot<PACKED, std::is_same<Act, ActF16>::value>(w, s, K, n, xrow);
+  return v;
+}
+
 // y = bf16( f32(bf16(g / (1 + exp(-g)))) * u ) on bf16 inputs g, u: SiLU in
 // fp32, rounded to bf16 first, then the product rounded once
 // (include/cudalm/kernels/qwen35_kernels.h:146-152).
@@ -142,18 +265,37 @@ __device__ __forceinline__ uint32_t silu_mul_bits(uint32_t g_bits, uint32_t u_bi
   return mul_bits(silu_bits(g_bits), u_bits);
 }
 
-// Prefill-chunk GEMM on 32 x 32 MFMA tiles (w4a16_gemm.hip): 32 activation
-// rows x 256 weight rows per 8-wave workgroup, any M, N and K % 128 == 0.
-template <bool PACKED>
+// GEMM of M >= 33 activation rows (w4a16_gemm.hip), the kernel chosen by
+// shape, for any N, M and K % 128 == 0.
+template <class Act, bool PACKED>
+int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
+                   int K, int M, hipStream_t stream);
+
+// Its 32 x 32 MFMA kernels alone: 32 activation rows x 256 weight rows per
+// 8-wave workgroup (at K = 1024 the split kernel).
+template <class Act, bool PACKED>
 int launch_prefill32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                      int K, int M, hipStream_t stream);
 
-// Waves per wave set of the K = 1024 split 32x32 kernel for an N x 1024 x M
-// GEMM on `cus` CUs, 0 when the unit GEMM serves the shape better.
-int prefill_split_waves(int N, int M, int cus, bool packed);
-
-// Registers per lane of that kernel at K = 1024 (prepacked instance).
+// Registers per lane of the split kernel at K = 1024 and of the unit GEMM
+// (prepacked instances).
 int prefill32_regs();
+int prefill_unit_regs();
+
+// GEMM on 64 x 64 wave tiles (w4a16_gemm_wide.hip), for M and N large enough
+// to give every CU a workgroup of 64 x 256 outputs.
+template <bool PACKED>
+bool wide_serves(int N, int K, int M);
+template <class Act, bool PACKED>
+int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
+                int M, hipStream_t stream);
+
+// The same kernel over gate and up, storing silu(gate) * up.
+bool wide_swiglu_serves(int N, int K, int M);
+template <bool PACKED>
+int launch_wide_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
+                       const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,
+                       hipStream_t stream);
 
 }  // namespace cudalm_hip
 

@@ -48,14 +48,6 @@
 namespace cudalm_hip {
 namespace {
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-// D = A (32 rows x 16 k) * B (16 k x 32 cols) + C, bf16 in, fp32 accumulate.
-__device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
 constexpr int kPB = kUnit * 16 + 1;  // LDS row pitch of one unit of x, 16-byte blocks (padded)
 
 template <int WVN, int MT>
@@ -65,7 +57,7 @@ constexpr size_t gemm32_lds_bytes() {
 
 // WVN waves along n, each owning NB 32-row weight tiles; MT 32-row
 // activation tiles per workgroup (every wave runs all of them).
-template <int WVN, int MT, int NB, bool PACKED, bool SVEC>
+template <class Act, int WVN, int MT, int NB, bool PACKED, bool SVEC>
 __global__ __launch_bounds__(WVN * 64) void w4a16_gemm32_kernel(
     const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
     const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int K, int M) {
@@ -185,7 +177,7 @@ __global__ __launch_bounds__(WVN * 64) void w4a16_gemm32_kernel(
 #pragma unroll
       for (int q = 0; q < CPW; ++q) {
         const int c = wave + q * WVN;
-        const f32x4_t o = group_offset(xo[q]);
+        const f32x4_t o = group_offset_t<Act>(xo[q]);
         if (c < NCH && i16 == 0) {
           const int gg = c / (2 * MT), st = c - gg * (2 * MT);
           *reinterpret_cast<f32x4_t*>(corr + gg * TM + st * 16 + 4 * a16) = o;
@@ -231,9 +223,9 @@ __global__ __launch_bounds__(WVN * 64) void w4a16_gemm32_kernel(
         for (int e = 0; e < 2; ++e) {
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) {
-            const u32x4_t B = decode_nibbles<PACKED>(e == 0 ? wl[nb][gg][d] : wh[nb][gg][d]);
+            const u32x4_t B = Act::template decode<PACKED>(e == 0 ? wl[nb][gg][d] : wh[nb][gg][d]);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) t[nb][mt] = mfma32(xa[d][e][mt], B, t[nb][mt]);
+            for (int mt = 0; mt < MT; ++mt) t[nb][mt] = mfma32<Act>(xa[d][e][mt], B, t[nb][mt]);
           }
         }
       }
@@ -273,10 +265,10 @@ __global__ __launch_bounds__(WVN * 64) void w4a16_gemm32_kernel(
         if (m < mrows) {
           // a NaN sum (infinite or NaN activations, overflow) is recomputed
           // by the reference loop, which keeps the reference's semantics
-          float v = 16.0f * acc[nb][mt][r];
+          float v = Act::kUnit * acc[nb][mt][r];
           if (__builtin_expect(v != v, 0))
-            v = w4a16_ref_dot<PACKED>(W, S, K, n, X + static_cast<size_t>(m0 + m) * K);
-          Y[static_cast<size_t>(m0 + m) * N + n] = static_cast<uint16_t>(f32_to_bf16_rne(v));
+            v = w4a16_ref_dot<PACKED, std::is_same<Act, ActF16>::value>(W, S, K, n, X + static_cast<size_t>(m0 + m) * K);
+          Y[static_cast<size_t>(m0 + m) * N + n] = static_cast<uint16_t>(Act::round(v));
         }
       }
   }
@@ -323,7 +315,7 @@ constexpr size_t gemm32_split_lds_bytes() {
                                        : static_cast<size_t>(WVN) * 64 * 16 * 4);
 }
 
-template <int WVN, bool PACKED, bool SVEC>
+template <class Act, int WVN, bool PACKED, bool SVEC>
 __global__ __launch_bounds__(WVN * 2 * 64) void w4a16_gemm32_split_kernel(
     const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
     const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int M) {
@@ -433,7 +425,7 @@ __global__ __launch_bounds__(WVN * 2 * 64) void w4a16_gemm32_split_kernel(
 #pragma unroll
     for (int q = 0; q < CPW; ++q) {
       const int c = wave + q * NW;
-      const f32x4_t o = group_offset(xo[q]);
+      const f32x4_t o = group_offset_t<Act>(xo[q]);
       if (c < NCH && i16 == 0)
         *reinterpret_cast<f32x4_t*>(corr + (c >> 1) * TM + (c & 1) * 16 + 4 * a16) = o;
     }
@@ -488,7 +480,7 @@ __global__ __launch_bounds__(WVN * 2 * 64) void w4a16_gemm32_split_kernel(
       for (int d = 0; d < 4; ++d)
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          acc = mfma32(xa[d][e], decode_nibbles<PACKED>(e == 0 ? wl[gq][d] : wh[gq][d]), acc);
+          acc = mfma32<Act>(xa[d][e], Act::template decode<PACKED>(e == 0 ? wl[gq][d] : wh[gq][d]), acc);
       t[gq] = acc;
     }
   }
@@ -533,15 +525,15 @@ __global__ __launch_bounds__(WVN * 2 * 64) void w4a16_gemm32_split_kernel(
   for (int r = 0; r < 16; ++r) {
     const int m = 8 * (r >> 2) + 4 * h + (r & 3);
     if (m < mrows) {
-      float val = 16.0f * total[r];
+      float val = Act::kUnit * total[r];
       if (__builtin_expect(val != val, 0))
-        val = w4a16_ref_dot<PACKED>(W, S, K, n, X + static_cast<size_t>(m0 + m) * K);
-      Y[static_cast<size_t>(m0 + m) * N + n] = static_cast<uint16_t>(f32_to_bf16_rne(val));
+        val = w4a16_ref_dot<PACKED, std::is_same<Act, ActF16>::value>(W, S, K, n, X + static_cast<size_t>(m0 + m) * K);
+      Y[static_cast<size_t>(m0 + m) * N + n] = static_cast<uint16_t>(Act::round(val));
     }
   }
 }
 
-template <int WVN, bool PACKED>
+template <class Act, int WVN, bool PACKED>
 int launch_gemm32_split(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                         int M, hipStream_t stream) {
   const size_t lds = gemm32_split_lds_bytes<WVN, PACKED>();
@@ -549,14 +541,14 @@ int launch_gemm32_split(const uint8_t* W, const uint16_t* S, const uint16_t* X, 
   const int gy = (M + 31) / 32;
   if (gy > 65535) return CUDALM_W4A16_ERANGE;
   const bool svec = !PACKED && aligned(S, 8);
-  auto kern = svec ? w4a16_gemm32_split_kernel<WVN, PACKED, true>
-                   : w4a16_gemm32_split_kernel<WVN, PACKED, false>;
+  auto kern = svec ? w4a16_gemm32_split_kernel<Act, WVN, PACKED, true>
+                   : w4a16_gemm32_split_kernel<Act, WVN, PACKED, false>;
   if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
   hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(WVN * 2 * 64), lds, stream, W, S, X, Y, N, M);
   return launch_status();
 }
 
-template <int WVN, int MT, int NB, bool PACKED>
+template <class Act, int WVN, int MT, int NB, bool PACKED>
 int launch_gemm32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                   int K, int M, hipStream_t stream) {
   const size_t lds = gemm32_lds_bytes<WVN, MT>();
@@ -564,26 +556,290 @@ int launch_gemm32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16
   const int gy = (M + 32 * MT - 1) / (32 * MT);
   if (gy > 65535) return CUDALM_W4A16_ERANGE;
   const bool svec = !PACKED && (K / kGroup) % 8 == 0 && aligned(S, 16);
-  auto kern = svec ? w4a16_gemm32_kernel<WVN, MT, NB, PACKED, true>
-                   : w4a16_gemm32_kernel<WVN, MT, NB, PACKED, false>;
+  auto kern = svec ? w4a16_gemm32_kernel<Act, WVN, MT, NB, PACKED, true>
+                   : w4a16_gemm32_kernel<Act, WVN, MT, NB, PACKED, false>;
   if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
   hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(WVN * 64), lds, stream, W, S, X, Y, N, K, M);
   return launch_status();
 }
 
-}  // namespace
+// ---------------------------------------------------------------------------
+// Unit GEMM kernel (prefill chunks): a k-slice of WV waves owns
+// TN = WV * RB * 16 weight rows and TM = CT * 16 activation rows. K is walked
+// one 8-group unit (1024 k) at a time: the unit's activations are staged
+// once into LDS (pair order), the slice computes the unit's offset table
+// once (waves split the chains), and every weight is decoded once, by the
+// wave that owns its rows, and feeds CT MFMA column tiles. Weights of a unit
+// are fetched up front (while the activations are staged). The per-output
+// operation sequence is the stream kernel's, so the bits are the same.
+//
+// KS > 1 k-slices split the units of the same output tile: slice s takes
+// units s, s + KS, ... with its own LDS buffers, keeps each unit partial,
+// and at the end the partials meet in LDS and are summed in unit order, so
+// the bits do not depend on KS. This serves few-tile, long-K shapes
+// (N = 1024, K = 2048 / 3584), where one slice would walk every unit alone.
+// ---------------------------------------------------------------------------
 
-template <bool PACKED>
-int launch_prefill32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
-                     int K, int M, hipStream_t stream) {
-  if (K == kUnit * kGroup) {
-    switch (prefill_split_waves(N, M, cu_count(), PACKED)) {
-      case 2: return launch_gemm32_split<2, PACKED>(W, S, X, Y, N, M, stream);
-      case 4: return launch_gemm32_split<4, PACKED>(W, S, X, Y, N, M, stream);
-      default: return launch_gemm32_split<8, PACKED>(W, S, X, Y, N, M, stream);
+constexpr int kSliceMaxUnits = 4;  // units per k-slice kept as partials (KS > 1)
+
+template <class Act, int RB, int CT, int WV, bool PACKED, bool SVEC, int KS = 1, bool IOFF = false>
+__global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
+    const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
+    const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int K, int M) {
+  constexpr int NT = WV * 64;  // threads of one k-slice
+  constexpr int TM = CT * 16;
+  constexpr int PB = x_pitch(kUnit * kGroup);  // LDS row pitch in 16-byte blocks (padded)
+  constexpr int NBLK = TM * kUnit * 16;  // 16-byte x blocks per unit
+  static_assert(NBLK % NT == 0, "staging must cover the tile exactly");
+  constexpr int BPT = NBLK / NT;  // x blocks staged per thread per unit
+  constexpr int XB = TM * PB;     // 16-byte blocks of one slice's x buffer
+  constexpr int NPART = KS == 1 ? 1 : kSliceMaxUnits;
+  extern __shared__ u32x4_t lds[];  // [KS][TM][PB] x, then [KS] offset tables
+
+  const int G = K >> 7;
+  const int U = (G + kUnit - 1) / kUnit;
+  const int ntiles = (N + kTileRows - 1) / kTileRows;
+  const int lane = threadIdx.x & 63;
+  const int slice = KS == 1 ? 0 : wave_id() / WV;
+  const int wave = wave_id() - slice * WV;  // wave within the slice
+  const int tid = static_cast<int>(threadIdx.x) - slice * NT;
+  const int i = lane & 15, a = lane >> 4;
+  const int m0 = blockIdx.y * TM;
+  const int mrows = min(TM, M - m0);
+  u32x4_t* xs = lds + slice * XB;
+  float* corr = reinterpret_cast<float*>(lds + KS * XB) + slice * (kUnit * CT * 16);
+
+  int rt[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) rt[rb] = min((blockIdx.x * WV + wave) * RB + rb, ntiles - 1);
+  const bool any_ok = (blockIdx.x * WV + wave) * RB < ntiles;
+
+  // lane addresses of each owned tile at group 0
+  const uint8_t* wbase[RB];
+  const uint8_t* sbase[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    if constexpr (PACKED) {
+      const uint8_t* tile = W + static_cast<size_t>(rt[rb]) * packed_tile_bytes(G);
+      wbase[rb] = tile + lane * 16;
+      sbase[rb] = tile + static_cast<size_t>(G) * 1024 + i * packed_scale_pitch(G);
+    } else {
+      const int row = min(rt[rb] * kTileRows + i, N - 1);
+      wbase[rb] = W + static_cast<size_t>(row) * (K >> 1) + a * 16;
+      sbase[rb] = reinterpret_cast<const uint8_t*>(S + static_cast<size_t>(row) * G);
     }
   }
-  return launch_gemm32<8, 1, 1, PACKED>(W, S, X, Y, N, K, M, stream);
+  constexpr int kStep = PACKED ? 1024 : 64;  // bytes between groups of one lane
+
+  const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  // KS == 1: the running unit sum; KS > 1: this slice's unit partials
+  f32x4_t acc[NPART][RB][CT];
+#pragma unroll
+  for (int q = 0; q < NPART; ++q)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) acc[q][rb][ct] = zero;
+
+  const int iters = (U + KS - 1) / KS;
+  for (int it = 0; it < iters; ++it) {
+    const int u = it * KS + slice;
+    const int uc = min(u, U - 1);  // a slice past the last unit re-reads it and skips the math
+    const int g0 = uc * kUnit;
+    const int gn = u < U ? min(kUnit, G - g0) : 0;
+    // the unit's activations first: they are staged and feed the offset
+    // table before any weight is used, and loads return in issue order
+    constexpr int RS = NT / (kUnit * 16);
+    static_assert(NT % (kUnit * 16) == 0, "a thread keeps one block column");
+    const int b = tid & (kUnit * 16 - 1);  // thread tid stages block b of rows tid / 128 + q * RS
+    const int r0 = tid / (kUnit * 16);
+    u32x4_t v[BPT];
+    {
+      const uint16_t* xcol = X + static_cast<size_t>(m0) * K + min(g0 * kGroup + 8 * b, K - 8);
+#pragma unroll
+      for (int q = 0; q < BPT; ++q)
+        v[q] = *reinterpret_cast<const u32x4_t*>(
+            xcol + static_cast<size_t>(min(r0 + q * RS, mrows - 1)) * K);
+    }
+    // then this unit's weights and scales (group indices clamped to G - 1)
+    u32x4_t w[RB][kUnit];
+    uint32_t sc[RB][kUnit / 2];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+      for (int gg = 0; gg < kUnit; ++gg)
+        w[rb][gg] = *reinterpret_cast<const u32x4_t*>(
+            wbase[rb] + static_cast<size_t>(min(g0 + gg, G - 1)) * kStep);
+      if constexpr (PACKED || SVEC) {
+        const u32x4_t sv = *reinterpret_cast<const u32x4_t*>(sbase[rb] + 2 * g0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sc[rb][q] = sv[q];
+      } else {
+        const uint16_t* srow = reinterpret_cast<const uint16_t*>(sbase[rb]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          sc[rb][q] = static_cast<uint32_t>(srow[min(g0 + 2 * q, G - 1)]) |
+                      (static_cast<uint32_t>(srow[min(g0 + 2 * q + 1, G - 1)]) << 16);
+      }
+    }
+    if (it > 0) __syncthreads();  // previous unit's readers are done
+    {
+      u32x4_t* xdst = xs + r0 * PB + x_slot(b);
+#pragma unroll
+      for (int q = 0; q < BPT; ++q) xdst[q * RS * PB] = pair_order(v[q]);
+    }
+    __syncthreads();
+    // offset table of the unit: chains (group, column tile) split over waves
+    // (IOFF: each wave runs the chains of its own groups inline instead, the
+    // same operands, and the table and its barrier are skipped)
+    if constexpr (!IOFF) {
+      for (int c = wave; c < kUnit * CT; c += WV) {
+        const int gg = c / CT, ct = c - gg * CT;
+        u32x4_t xa[4];
+        load_group_x(xa, xs + (ct * 16 + i) * PB + gg * 16, a);
+        const f32x4_t o = group_offset_t<Act>(xa);
+        if (i == 0) *reinterpret_cast<f32x4_t*>(corr + c * 16 + 4 * a) = o;
+      }
+      __syncthreads();
+    }
+    if (!any_ok) continue;
+
+    f32x4_t part[RB][CT];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) part[rb][ct] = zero;
+    // one group: offset-seeded weight chains, then the scale fma into part
+    auto group = [&](int gg) {
+      u32x4_t xa[CT][4];
+      f32x4_t t[RB][CT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        load_group_x(xa[ct], xs + (ct * 16 + i) * PB + gg * 16, a);
+        const f32x4_t o = IOFF ? group_offset_t<Act>(xa[ct])
+                               : *reinterpret_cast<const f32x4_t*>(corr + (gg * CT + ct) * 16 + 4 * a);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) t[rb][ct] = o;
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const u32x4_t B = Act::template decode<PACKED>(w[rb][gg][d]);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) t[rb][ct] = Act::mma(xa[ct][d], B, t[rb][ct]);
+        }
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const float s = half_bits_to_f32((sc[rb][gg >> 1] >> (16 * (gg & 1))) & 0xFFFFu);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            part[rb][ct][r] = __builtin_fmaf(s, t[rb][ct][r], part[rb][ct][r]);
+      }
+    };
+    if (gn == kUnit) {
+      // full unit: straight-line, so independent group chains interleave
+#pragma unroll
+      for (int gg = 0; gg < kUnit; ++gg) group(gg);
+    } else {
+#pragma unroll
+      for (int gg = 0; gg < kUnit; ++gg)
+        if (gg < gn) group(gg);
+    }
+    if constexpr (KS == 1) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) acc[0][rb][ct] = acc[0][rb][ct] + part[rb][ct];
+    } else {
+#pragma unroll
+      for (int q = 0; q < NPART; ++q)
+        if (q == it)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) acc[q][rb][ct] = part[rb][ct];
+    }
+  }
+
+  f32x4_t total[RB][CT];
+  if constexpr (KS == 1) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) total[rb][ct] = acc[0][rb][ct];
+  } else {
+    // unit partials meet in LDS (over the x buffers): slot [u][wave][rb][ct][lane]
+    __syncthreads();
+    f32x4_t* slots = reinterpret_cast<f32x4_t*>(lds);
+    if (any_ok) {
+#pragma unroll
+      for (int q = 0; q < NPART; ++q) {
+        const int u = q * KS + slice;
+        if (q < iters && u < U)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+              slots[(((u * WV + wave) * RB + rb) * CT + ct) * 64 + lane] = acc[q][rb][ct];
+      }
+    }
+    __syncthreads();
+    if (slice != 0) return;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        total[rb][ct] = zero;
+        for (int u = 0; u < U; ++u)
+          total[rb][ct] = total[rb][ct] + slots[(((u * WV + wave) * RB + rb) * CT + ct) * 64 + lane];
+      }
+  }
+  if (!any_ok) return;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int n = ((blockIdx.x * WV + wave) * RB + rb) * kTileRows + i;
+    if (n >= N) continue;
+    uint16_t* col = Y + static_cast<size_t>(m0 + 4 * a) * N + n;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (ct * 16 + 4 * a + r < mrows)
+          col[static_cast<size_t>(ct * 16 + r) * N] = static_cast<uint16_t>(Act::round(
+              out_value<Act, PACKED>(total[rb][ct][r], W, S, K, n,
+                                         X + static_cast<size_t>(m0 + ct * 16 + 4 * a + r) * K)));
+  }
+}
+
+template <class Act, int RB, int CT, int WV, bool PACKED, int KS = 1, bool IOFF = false>
+int launch_gemm_unit(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
+                     int K, int M, hipStream_t stream) {
+  constexpr int TM = CT * 16;
+  const size_t xbytes = static_cast<size_t>(TM) * x_pitch(kUnit * kGroup) * 16;
+  const size_t lds = KS * (xbytes + static_cast<size_t>(kUnit) * CT * 16 * sizeof(float));
+  const int G = K / kGroup;
+  if constexpr (KS > 1) {
+    // every slice keeps at most kSliceMaxUnits partials, and all of them
+    // must fit the x buffers they are parked in
+    const int U = (G + kUnit - 1) / kUnit;
+    if (U > KS * kSliceMaxUnits ||
+        static_cast<size_t>(U) * WV * RB * CT * 64 * 16 > KS * xbytes)
+      return launch_gemm_unit<Act, RB, CT, WV, PACKED, 1, IOFF>(W, S, X, Y, N, K, M, stream);
+  }
+  const int ntiles = (N + kTileRows - 1) / kTileRows;
+  const int gx = (ntiles + WV * RB - 1) / (WV * RB);
+  const int gy = (M + TM - 1) / TM;
+  if (gy > 65535) return CUDALM_W4A16_ERANGE;
+  const bool svec = !PACKED && G % 8 == 0 && aligned(S, 16);
+  auto kern = svec ? w4a16_gemm_unit_kernel<Act, RB, CT, WV, PACKED, true, KS, IOFF>
+                   : w4a16_gemm_unit_kernel<Act, RB, CT, WV, PACKED, false, KS, IOFF>;
+  if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
+  hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(WV * KS * 64), lds, stream, W, S, X, Y, N, K, M);
+  return launch_status();
 }
 
 // Waves per wave set of the K = 1024 split kernel: the narrowest of 2, 4
@@ -607,11 +863,67 @@ int prefill_split_waves(int N, int M, int cus, bool packed) {
   return 0;
 }
 
-int prefill32_regs() { return regs_of(w4a16_gemm32_split_kernel<8, true, false>); }
+}  // namespace
 
-template int launch_prefill32<true>(const uint8_t*, const uint16_t*, const uint16_t*, uint16_t*,
-                                    int, int, int, hipStream_t);
-template int launch_prefill32<false>(const uint8_t*, const uint16_t*, const uint16_t*, uint16_t*,
-                                     int, int, int, hipStream_t);
+template <class Act, bool PACKED>
+int launch_prefill32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
+                     int K, int M, hipStream_t stream) {
+  if (K == kUnit * kGroup) {
+    switch (prefill_split_waves(N, M, cu_count(), PACKED)) {
+      case 2: return launch_gemm32_split<Act, 2, PACKED>(W, S, X, Y, N, M, stream);
+      case 4: return launch_gemm32_split<Act, 4, PACKED>(W, S, X, Y, N, M, stream);
+      default: return launch_gemm32_split<Act, 8, PACKED>(W, S, X, Y, N, M, stream);
+    }
+  }
+  return launch_gemm32<Act, 8, 1, 1, PACKED>(W, S, X, Y, N, K, M, stream);
+}
+
+// Prefill chunks (M >= 33). Shapes with enough 64 x 256 output tiles take
+// the wide kernel (wide_serves). The 32 x 32 MFMA GEMM (32 activation rows x
+// 256 weight rows per 8-wave workgroup) serves K <= 1024
+// when its workgroups fill between 3/4 and all of the CUs in one round
+// (3584x1024 and 4096x1024 at M = 512: 10.3 -> 9.6-9.9 us, 10.7 -> 9.5-10.0 us);
+// elsewhere the 16 x 16 unit GEMM is faster (one round of 32 x 256 tiles
+// leaves too many CUs idle below that, and past one round it takes two).
+// Unit GEMM tiles: 128 x 32 of 8 waves while they fill most of the CUs,
+// else 64 x 32 of 4 waves, with two k-slices of 4 waves when K spans
+// several units (1024x3584 at M = 512: 16.7 -> 14.6 us). The 4-wave tiles
+// run their offset chains inline (512x1024x512 5.8 -> 5.5 us, 1024x3584x512
+// 14.4 -> 13.8 us); inline chains cost the 8-wave tiles 0.6 us at
+// 3584x1024x512, so those keep the table.
+template <class Act, bool PACKED>
+int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
+                   int M, hipStream_t stream) {
+  const int cus = cu_count();
+  if (wide_serves<PACKED>(N, K, M)) return launch_wide<Act, PACKED>(W, S, X, Y, N, K, M, stream);
+  if (K == kUnit * kGroup && prefill_split_waves(N, M, cus, PACKED) != 0)
+    return launch_prefill32<Act, PACKED>(W, S, X, Y, N, K, M, stream);
+  if (K < kUnit * kGroup) {
+    const long long wgs32 = static_cast<long long>((N + 255) / 256) * ((M + 31) / 32);
+    if (4 * wgs32 >= 3LL * cus && wgs32 <= cus)
+      return launch_prefill32<Act, PACKED>(W, S, X, Y, N, K, M, stream);
+  }
+  const long long wgs = static_cast<long long>((N + 127) / 128) * ((M + 31) / 32);
+  // (crossover measured between 128 and 168 workgroups of 128 x 32:
+  // 2048x1024x256 5.7 vs 6.9 us, 3584x1024x192 7.4 vs 6.9 us)
+  if (5 * wgs >= 3LL * cus) return launch_gemm_unit<Act, 1, 2, 8, PACKED>(W, S, X, Y, N, K, M, stream);
+  if (K > kUnit * kGroup)
+    return launch_gemm_unit<Act, 1, 2, 4, PACKED, 2, true>(W, S, X, Y, N, K, M, stream);
+  return launch_gemm_unit<Act, 1, 2, 4, PACKED, 1, true>(W, S, X, Y, N, K, M, stream);
+}
+
+int prefill32_regs() { return regs_of(w4a16_gemm32_split_kernel<ActBf16, 8, true, false>); }
+int prefill_unit_regs() { return regs_of(w4a16_gemm_unit_kernel<ActBf16, 1, 2, 8, true, false>); }
+
+#define W4A16_PREFILL(ACT, PACKED)                                                             \
+  template int launch_prefill32<ACT, PACKED>(const uint8_t*, const uint16_t*, const uint16_t*, \
+                                             uint16_t*, int, int, int, hipStream_t);           \
+  template int launch_prefill<ACT, PACKED>(const uint8_t*, const uint16_t*, const uint16_t*,   \
+                                           uint16_t*, int, int, int, hipStream_t)
+W4A16_PREFILL(ActBf16, true);
+W4A16_PREFILL(ActBf16, false);
+W4A16_PREFILL(ActF16, true);
+W4A16_PREFILL(ActF16, false);
+#undef W4A16_PREFILL
 
 }  // namespace cudalm_hip

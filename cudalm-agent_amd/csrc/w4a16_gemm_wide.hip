@@ -1,0 +1,597 @@
+// W4A16 GEMM on 64 x 64 wave tiles (MI355X, gfx950): prefill chunks and
+// scoring calls whose outputs fill the chip with 64 x 256 tiles, and the
+// SwiGLU front half of an MLP for such chunks.
+//
+// Contract (reference: tests/cuda/test_int4_gemv_bf16.cpp:54-69 applied row
+// by row):  y[m,n] = rne( sum_k q[n,k] * f32(s[n,k/128]) * f32(x[m,k]) ).
+//
+// What bounds it. One decoded weight dword (7-8 VALU) feeds MT = 2 MFMAs of
+// 32 x 32 x 16, and one 16-byte activation read feeds NT = 2; per group a
+// wave issues 32 MFMAs (1056 cycles at the measured 33 cycles each) beside
+// ~220 VALU, 28 LDS reads and 4 LDS writes. With two workgroups of 4 waves
+// per CU (<= 256 registers) a pair of groups takes ~4850 cycles for both, 87%
+// of the matrix cores' issue rate; one workgroup alone takes ~4280, so the
+// kernel needs both. The rest of a workgroup's ~26,000 cycles at K = 1024 is
+// the first loads (~2,900) and the stores (~3,500), which overlap the other
+// workgroup's groups. Under this load the part lowers its clock to ~1.65 GHz
+// (the same launch on all-zero data runs 1.24x faster), as it does for a
+// large library GEMM (1.42 PFLOP/s measured for 8192^3 bf16).
+//
+// Measured against the 128 x 32 unit GEMM and the split 32 x 32 kernel, which
+// serve the smaller shapes (same box, prepacked / file layout, us):
+//   6144 x 1024, M = 2048:  42.3 -> 29.8 / 46.8 -> 32.3
+//   4096 x 1024, M = 1024:  16.0 -> 13.4 / 17.4 -> 14.3
+//   248320 x 1024, M = 256:  292 -> 147 / 279 -> 175
+//   4096 x 4096, M = 1024:  55.5 -> 45.6 (64 x 32 wave tiles)
+//   SwiGLU 3584 x 1024, M = 1000: 143.5 (32-row chunks) -> 22.3 / 143 -> 23.0
+// Wave tiles of 128 x 64 and 64 x 128 outputs with one wave per SIMD (400-470
+// registers) measured 1.4-1.5x slower: nothing covers a wave's own latencies.
+// 128 x 32 tiles of 8 waves: 1.2x slower (one activation read per MFMA).
+//
+// Same bits as every other kernel of the library: per group the offset chain
+// (four 16 x 16 x 32 MFMAs of x against -1.5) seeds the weight chain, run as
+// 32 x 32 x 16 half steps in the order of w4a16_gemm.hip, then
+// part = fma(s[n, g], tmp, part) in group order from 0 within an 8-group unit
+// and total = 0 + part_u in unit order.
+//
+// Work decomposition. A workgroup of WV waves owns 32 MT activation rows and
+// WV x 32 NT weight rows, each wave its own weight rows. x of a group is
+// staged into one of four LDS buffers two groups ahead (loads to registers
+// three ahead), with one barrier per two groups; the wave that stages 16 rows
+// also runs their offset chains. Weights and scales are loaded one group
+// ahead into registers. The operands of a 16-k step are read and decoded
+// during the step before, pinned there by scheduling barriers: left alone
+// the compiler reads them just in time.
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "cudalm_w4a16.h"
+#include "hip_common.h"
+#include "w4a16_device.h"
+
+namespace cudalm_hip {
+namespace {
+
+// A buffer resource over everything from a uniform base on: loads take a
+// 32-bit lane offset and a scalar offset, so walking the groups costs no
+// vector address arithmetic and no 64-bit lane pointers. Every offset used
+// is inside the operand it addresses.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xFFFFFFFFu, 0x00020000);
+}
+__device__ __forceinline__ u32x4_t load_b128(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
+}
+
+constexpr int kWidePitch = 17;  // 16-byte blocks per LDS row of one group (padded)
+
+template <int MT>
+constexpr size_t wide_lds_bytes() {
+  return static_cast<size_t>(4) * 32 * MT * (kWidePitch * 16 + 4);
+}
+
+// What a wave multiplies: one weight matrix, or the gate and up matrices.
+struct WideArgs {
+  const uint8_t* w[2];
+  const uint16_t* s[2];
+  const uint16_t* x;
+  uint16_t* y;
+  int N, K, M;
+  int tiles_m, tiles_n;
+};
+
+// SVEC: 4-byte aligned scale pairs (prepacked, or G even and S 4 B aligned)
+template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU>
+__global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs p) {
+  static_assert(!GLU || NT == 2, "a wave holds a gate and an up tile");
+  constexpr int BM = 32 * MT;
+  constexpr int BNW = GLU ? 32 : 32 * NT;  // output columns per wave
+  constexpr int NS = BM / 16;              // 16-row staging slices
+  constexpr int SPW = (NS + WV - 1) / WV;  // slices per wave
+  extern __shared__ u32x4_t lds[];
+  constexpr int XB = BM * kWidePitch;  // 16-byte blocks of one group's x
+  float* const ob = reinterpret_cast<float*>(lds + 4 * XB);
+
+  const int K = p.K, N = p.N;
+  const int G = K >> 7;
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();
+  const int j = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, a16 = lane >> 4;
+
+  // tile order: each XCD (workgroup L runs on XCD L % 8) takes a contiguous
+  // run of tiles, in bands of 8 tile rows walked column by column
+  int bm, bn;
+  {
+    const int total = p.tiles_m * p.tiles_n;
+    const int per = (total + 7) >> 3;
+    const int L = blockIdx.x;
+    const int idx = (L & 7) * per + (L >> 3);
+    if ((L >> 3) >= per || idx >= total) return;
+    const int band = 8 * p.tiles_n;
+    const int bi = idx / band;
+    const int rem = idx - bi * band;
+    const int rows = min(8, p.tiles_m - bi * 8);
+    bn = rem / rows;
+    bm = bi * 8 + rem - bn * rows;
+  }
+  const int m0 = bm * BM;
+  const int mrows = min(BM, p.M - m0);
+  const int nbase = (bn * WV + wave) * BNW;
+  const bool wave_ok = nbase < N;
+
+  // staging: wave w stages slices w, w + WV, ...: load q of slice s reads
+  // row 16 s + 4 q + lane / 16, block lane % 16 of the group
+  const auto xsrc = make_rsrc(p.x + static_cast<size_t>(m0) * K);
+  int xoff[SPW][4];
+#pragma unroll
+  for (int sl = 0; sl < SPW; ++sl)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      xoff[sl][q] = min(16 * (wave + sl * WV) + 4 * q + a16, mrows - 1) * K * 2 + 16 * i16;
+
+  // weights: a base per wave (uniform) and 32-bit lane offsets from it
+  const int nfirst = min(nbase, N - 1);
+  const size_t wfirst = PACKED ? static_cast<size_t>(nfirst >> 4) * packed_tile_bytes(G)
+                               : static_cast<size_t>(nfirst) * (K >> 1);
+  const auto wsrc0 = make_rsrc(p.w[0] + wfirst);
+  const auto wsrc1 = make_rsrc((GLU ? p.w[1] : p.w[0]) + wfirst);
+  const auto ssrc0 = PACKED ? wsrc0 : make_rsrc(p.s[0] + static_cast<size_t>(nfirst) * G);
+  const auto ssrc1 = PACKED ? wsrc1 : make_rsrc((GLU ? p.s[1] : p.s[0]) + static_cast<size_t>(nfirst) * G);
+  int woff[NT], soff[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = min(nbase + (GLU ? 0 : 32 * nt) + j, N - 1);
+    if constexpr (PACKED) {
+      const int tile = ((n >> 4) - (nfirst >> 4)) * static_cast<int>(packed_tile_bytes(G));
+      woff[nt] = tile + 16 * (16 * h + (n & 15));
+      soff[nt] = tile + G * 1024 + (n & 15) * packed_scale_pitch(G);
+    } else {
+      woff[nt] = (n - nfirst) * (K >> 1) + 16 * h;
+      soff[nt] = (n - nfirst) * G * 2;
+    }
+  }
+  constexpr int kStep = PACKED ? 1024 : 64;  // bytes between groups of one lane
+  constexpr int kHi = PACKED ? 512 : 32;     // lane chunk 2 + h after chunk h
+
+  u32x4_t xr[SPW][4];
+  auto load_x = [&](int g) {
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) xr[sl][q] = load_b128(xsrc, xoff[sl][q], g * (kGroup * 2));
+  };
+  // Staging of the next group's x, in pieces that the group loop places
+  // between its steps: the wave's slice rows go to LDS in pair order
+  // (stage_write), come back in MFMA operand layout (stage_read; only this
+  // wave writes and reads them here), feed the offset chain one step at a
+  // time (stage_chain), and the chain's result goes to the table.
+  u32x4_t xo[SPW][2];
+  f32x4_t oc[SPW];
+  auto slice_ok = [&](int sl) { return NS % WV == 0 || wave + sl * WV < NS; };
+  auto stage_write = [&](u32x4_t* xb) {
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+      if (slice_ok(sl))
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          xb[(16 * (wave + sl * WV) + 4 * q + a16) * kWidePitch + i16] = pair_order(xr[sl][q]);
+  };
+  auto stage_read = [&](const u32x4_t* xb, int d) {
+    if (d == 0) wave_lds_sync();
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+      xo[sl][d & 1] = xb[(16 * min(wave + sl * WV, NS - 1) + i16) * kWidePitch + 4 * a16 + d];
+  };
+  auto stage_chain = [&](int d) {
+    const u32x4_t neg = {Act::kNegOffsetPair, Act::kNegOffsetPair, Act::kNegOffsetPair,
+                         Act::kNegOffsetPair};
+    const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl) oc[sl] = Act::mma(xo[sl][d & 1], neg, d == 0 ? zero : oc[sl]);
+  };
+  auto stage_table = [&](float* ob) {
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+      if (slice_ok(sl))  // every column of the chain's tile holds the same values
+        *reinterpret_cast<f32x4_t*>(ob + 16 * (wave + sl * WV) + 4 * a16) = oc[sl];
+  };
+
+  struct WBuf {
+    u32x4_t lo[NT], hi[NT];
+  };
+  auto load_w = [&](WBuf& b, int g) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      b.lo[nt] = load_b128(nt == 0 || !GLU ? wsrc0 : wsrc1, woff[nt], g * kStep);
+      b.hi[nt] = load_b128(nt == 0 || !GLU ? wsrc0 : wsrc1, woff[nt] + kHi, g * kStep);
+    }
+  };
+  // scales of groups g, g + 1 (g even)
+  auto load_s = [&](uint32_t (&sc)[NT], int g) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const auto src = nt == 0 || !GLU ? ssrc0 : ssrc1;
+      if constexpr (PACKED || SVEC)
+        sc[nt] = __builtin_amdgcn_raw_buffer_load_b32(src, soff[nt], 2 * g, 0);
+      else
+        sc[nt] = __builtin_amdgcn_raw_buffer_load_b16(src, soff[nt], 2 * g, 0) |
+                 (static_cast<uint32_t>(
+                      __builtin_amdgcn_raw_buffer_load_b16(src, soff[nt], 2 * min(g + 1, G - 1), 0))
+                  << 16);
+    }
+  };
+
+  const f32x16_t zero16 = {};
+  f32x16_t part[MT][NT];
+  f32x16_t acc[MULTI ? MT : 1][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      part[mt][nt] = zero16;
+      if constexpr (MULTI) acc[mt][nt] = zero16;
+    }
+
+  // One group: eight 16-k steps, the operands of a step read and decoded
+  // during the step before. between(s) runs beside step s.
+  auto group = [&](const u32x4_t* xb, const float* ob, const WBuf& b, const uint32_t (&sc)[NT],
+                   int odd, auto&& between, auto&& tail) {
+    const u32x4_t* xa = xb + j * kWidePitch + 4 * h;
+    u32x4_t A[2][MT], B[2][NT];
+    auto fetch = [&](int s) {
+      const int d = s >> 1, e = s & 1;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) A[s & 1][mt] = xa[mt * 32 * kWidePitch + 8 * e + d];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        B[s & 1][nt] = Act::template decode<PACKED>(e == 0 ? b.lo[nt][d] : b.hi[nt][d]);
+    };
+    fetch(0);
+    f32x16_t t[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const float* cr = ob + mt * 32 + 4 * h;
+      f32x16_t o;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4_t o4 = *reinterpret_cast<const f32x4_t*>(cr + 8 * q);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[4 * q + r] = o4[r];
+      }
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) t[mt][nt] = o;
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (s < 7) fetch(s + 1);
+      between(s);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) t[mt][nt] = mfma32<Act>(A[s & 1][mt], B[s & 1][nt], t[mt][nt]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    tail();
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      float s = half_bits_to_f32((sc[nt] >> (16 * odd)) & 0xFFFFu);
+      asm("" : "+v"(s));  // keeps v_fma_f32: v_fma_mix_f32 on the fp16 bits issues at a lower rate
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          part[mt][nt][r] = __builtin_fmaf(s, t[mt][nt][r], part[mt][nt][r]);
+    }
+  };
+
+  WBuf w0, w1;
+  uint32_t sc[NT], scn[NT];
+  const auto fold = [&] {
+    if constexpr (MULTI) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          acc[mt][nt] = acc[mt][nt] + part[mt][nt];
+          part[mt][nt] = zero16;
+        }
+    }
+  };
+  // prologue: the first two groups of x, then the first weights
+  {
+    load_x(0);
+    u32x4_t x0[SPW][4];
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x0[sl][q] = xr[sl][q];
+    load_x(min(1, G - 1));
+    u32x4_t x1[SPW][4];
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        x1[sl][q] = xr[sl][q];
+        xr[sl][q] = x0[sl][q];
+      }
+    load_w(w0, 0);
+    load_s(sc, 0);
+    stage_write(lds);
+#pragma unroll
+    for (int sl = 0; sl < SPW; ++sl)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) xr[sl][q] = x1[sl][q];
+    stage_write(lds + XB);
+    load_x(min(2, G - 1));
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        stage_read(lds + q * XB, d);
+        stage_chain(d);
+      }
+      stage_table(ob + q * BM);
+    }
+  }
+  __syncthreads();
+  int g = 0, cur = 0;
+  for (; g + 1 < G; g += 2, cur ^= 2) {
+    // groups g and g + 1 from one buffer pair, g + 2 and g + 3 staged into
+    // the other meanwhile
+    const int nxt = cur ^ 2;
+    group(lds + cur * XB, ob + cur * BM, w0, sc, 0, [&](int s) {
+      if (s == 0) stage_write(lds + nxt * XB);
+      if (s == 1) load_x(min(g + 3, G - 1));
+      if (s == 1) load_w(w1, g + 1);
+      if (s == 1) load_s(scn, min(g + 2, (G - 1) & ~1));
+      if (s >= 3 && s < 7) stage_chain(s - 3);
+      if (s >= 2 && s < 6) stage_read(lds + nxt * XB, s - 2);
+      if (s == 7) stage_table(ob + nxt * BM);
+    }, [] {});
+    group(lds + cur * XB + XB, ob + cur * BM + BM, w1, sc, 1, [&](int s) {
+      if (s == 0) stage_write(lds + nxt * XB + XB);
+      if (s == 1) load_x(min(g + 4, G - 1));
+      if (s == 1) load_w(w0, min(g + 2, G - 1));
+      if (s >= 3 && s < 7) stage_chain(s - 3);
+      if (s >= 2 && s < 6) stage_read(lds + nxt * XB + XB, s - 2);
+      if (s == 7) stage_table(ob + nxt * BM + BM);
+    }, [] { __syncthreads(); });
+    if (MULTI && (g & 7) == 6) fold();
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) sc[nt] = scn[nt];
+  }
+  if (g < G) group(lds + cur * XB, ob + cur * BM, w0, sc, 0, [](int) {}, [] {});
+  if (MULTI && (G & 7) != 0) fold();
+  // every wave is done with the staged x; from here on each wave has its own
+  // part of the LDS
+  __syncthreads();
+  if (!wave_ok) return;
+  constexpr bool F16 = std::is_same<Act, ActF16>::value;
+  constexpr int kOutPitch = BNW + 8;  // 16-bit elements per LDS output row (padded)
+  static_assert(static_cast<size_t>(WV) * BM * kOutPitch * 2 <= wide_lds_bytes<MT>(), "fits");
+  uint16_t* const ot = reinterpret_cast<uint16_t*>(lds) + wave * BM * kOutPitch;
+  const uint32_t psel = (j & 1) ? 0x03020706u : 0x05040100u;  // v_perm_b32 over (other:own)
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    // one unit: total = 0 + part; kUnit * total in one exact fma
+    f32x16_t v[NT];
+    bool bad = false;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      v[nt] = MULTI ? acc[MULTI ? mt : 0][nt] : part[mt][nt];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[nt][r] = __builtin_fmaf(Act::kUnit, v[nt][r], 0.0f);
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) bad |= __builtin_isunordered(v[nt][r], v[nt][r + 1]);
+    }
+    // Rows r and r + 1 of column j are one dword; neighbouring lanes swap
+    // theirs so that the even lane writes row r, the odd one row r + 1, both
+    // columns of the pair (16-bit LDS writes cost as many LDS cycles each).
+    uint16_t* const pair =
+        ot + (mt * 32 + 4 * h + (j & 1)) * kOutPitch + (j & ~1);
+#pragma unroll
+    for (int r = 0; r < 16; r += 2)
+#pragma unroll
+      for (int nt = 0; nt < (GLU ? 1 : NT); ++nt) {
+        uint32_t own;
+        if constexpr (GLU)
+          own = silu_mul_bits(f32_to_bf16_rne(v[0][r]), f32_to_bf16_rne(v[1][r])) |
+                silu_mul_bits(f32_to_bf16_rne(v[0][r + 1]), f32_to_bf16_rne(v[1][r + 1])) << 16;
+        else
+          own = Act::round2(v[nt][r], v[nt][r + 1]);
+        const uint32_t other = static_cast<uint32_t>(
+            __builtin_amdgcn_mov_dpp(static_cast<int>(own), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+        // even: own.lo | other.lo << 16; odd: other.hi | own.hi << 16
+        *reinterpret_cast<uint32_t*>(pair + (8 * (r >> 2) + (r & 3)) * kOutPitch + 32 * nt) =
+            __builtin_amdgcn_perm(other, own, psel);
+      }
+    if (__builtin_expect(bad, 0)) {
+      // outputs whose fast sum is NaN: the reference loop's value instead
+      wave_lds_sync();
+      for (int q = 0; q < 16 * NT; ++q) {
+        const int r = q & 15, nt = q >> 4;
+        const int m = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        const int n = nbase + (GLU ? 0 : 32 * nt) + j;
+        if (m >= mrows || n >= N) continue;
+        float f[NT];
+#pragma unroll
+        for (int c = 0; c < NT; ++c) {
+          f[c] = v[c][0];
+#pragma unroll
+          for (int e = 1; e < 16; ++e) f[c] = r == e ? v[c][e] : f[c];
+        }
+        const uint16_t* xrow = p.x + static_cast<size_t>(m0 + m) * K;
+        if constexpr (GLU) {
+          const float own = nt == 0 ? f[0] : f[1];
+          if (own == own) continue;
+          const float e = w4a16_ref_dot<PACKED>(p.w[nt], p.s[nt], K, n, xrow);
+          // gate first (q ascending): up's turn recomputes gate if it was NaN too
+          float g = nt == 0 ? e : f[0];
+          const float u = nt == 0 ? f[1] : e;
+          if (g != g && nt == 1) g = w4a16_ref_dot<PACKED>(p.w[0], p.s[0], K, n, xrow);
+          ot[m * kOutPitch + j] =
+              static_cast<uint16_t>(silu_mul_bits(f32_to_bf16_rne(g), f32_to_bf16_rne(u)));
+        } else {
+          float own = f[0];
+#pragma unroll
+          for (int c = 1; c < NT; ++c) own = nt == c ? f[c] : own;
+          if (own != own)
+            ot[m * kOutPitch + 32 * nt + j] = static_cast<uint16_t>(
+                Act::round(w4a16_ref_dot<PACKED, F16>(p.w[0], p.s[0], K, n, xrow)));
+        }
+      }
+    }
+  }
+  wave_lds_sync();
+  // rows out: 16 bytes per lane where every row of y starts 16 B aligned,
+  // else one output per lane
+  uint16_t* const yt = p.y + static_cast<size_t>(m0) * N + nbase;
+  const int ncols = min(BNW, N - nbase);
+  if ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0) {
+    constexpr int LPR = BNW / 8;   // lanes per row
+    constexpr int RPI = 64 / LPR;  // rows per store
+    const int c = 8 * (lane % LPR), r0 = lane / LPR;
+    if (c < ncols) {
+#pragma unroll
+      for (int r = 0; r < BM; r += RPI)
+        if (r + r0 < mrows)
+          *reinterpret_cast<u32x4_t*>(yt + static_cast<size_t>(r + r0) * N + c) =
+              *reinterpret_cast<const u32x4_t*>(ot + (r + r0) * kOutPitch + c);
+    }
+  } else {
+    constexpr int RPI = 64 / (BNW < 64 ? BNW : 64);
+    const int c0 = lane % (BNW < 64 ? BNW : 64), r0 = lane / (BNW < 64 ? BNW : 64);
+    for (int r = r0; r < mrows; r += RPI)
+#pragma unroll
+      for (int c = c0; c < BNW; c += 64)
+        if (c < ncols) yt[static_cast<size_t>(r) * N + c] = ot[r * kOutPitch + c];
+  }
+}
+
+template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU>
+int launch_wide_t(WideArgs p, hipStream_t stream) {
+  constexpr int BN = WV * (GLU ? 32 : 32 * NT);
+  p.tiles_m = (p.M + 32 * MT - 1) / (32 * MT);
+  p.tiles_n = (p.N + BN - 1) / BN;
+  auto kern = w4a16_gemm_wide_kernel<Act, MT, NT, WV, OCC, PACKED, SVEC, MULTI, GLU>;
+  const size_t lds = wide_lds_bytes<MT>();
+  if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
+  const int grid = 8 * ((p.tiles_m * p.tiles_n + 7) / 8);  // an equal run of tiles per XCD
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(WV * 64), lds, stream, p);
+  return launch_status();
+}
+
+// Tiles of BM x BN outputs, -1 beyond the kernel's index ranges (32-bit tile
+// numbers and lane offsets; M as in the other prefill kernels' grids).
+long long wide_tiles(int N, int K, int M, int bm, int bn) {
+  if (K > (1 << 20) || M > 65535 * 32) return -1;
+  const long long t = static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  return t < (1LL << 30) ? t : -1;
+}
+
+}  // namespace
+
+// Where the 64 x 256 tiles beat the smaller-tiled prefill kernels (both in
+// us, theirs first; t = tiles on 256 CUs). Prepacked: from 25/32 of a tile
+// per CU: K = 1024 t = 182 12.2 / 12.4, 192 12.2 / 12.5, 208 15.0 / 12.8, 312
+// 19.1 / 18.7, 768 42.3 / 29.8; K = 3584 t = 112 25.2 / 25.6, 208 44.6 / 35.0.
+// File layout, whose loads the smaller tiles repeat more often: from 5/8 at
+// K <= 1024 (t = 128 9.6 / 9.7, 182 14.1 / 13.2, 768 46.8 / 32.3) and from 3/8
+// beyond (K = 2048 t = 96 17.0 / 15.5, 64 11.5 / 13.8; K = 3584 t = 104 33.6 /
+// 25.7).
+template <bool PACKED>
+bool wide_serves(int N, int K, int M) {
+  const long long t = wide_tiles(N, K, M, 64, 256);
+  const long long need = PACKED ? 25 : K <= kUnit * kGroup ? 20 : 12;  // 32nds of a tile per CU
+  return t >= 0 && 32 * t >= need * cu_count();
+}
+
+template <class Act, bool PACKED>
+int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
+                int M, hipStream_t stream) {
+  WideArgs p = {};
+  p.w[0] = p.w[1] = W;
+  p.s[0] = p.s[1] = S;
+  p.x = X;
+  p.y = Y;
+  p.N = N;
+  p.K = K;
+  p.M = M;
+  const bool svec = PACKED || ((K / kGroup) % 2 == 0 && aligned(S, 4));
+  if (K <= kUnit * kGroup) {
+    if constexpr (!PACKED)
+      if (!svec) return launch_wide_t<Act, 2, 2, 4, 2, PACKED, false, false, false>(p, stream);
+    return launch_wide_t<Act, 2, 2, 4, 2, PACKED, true, false, false>(p, stream);
+  }
+  if constexpr (!PACKED)
+    if (!svec) return launch_wide_t<Act, 2, 1, 4, 2, PACKED, false, true, false>(p, stream);
+  return launch_wide_t<Act, 2, 1, 4, 2, PACKED, true, true, false>(p, stream);
+}
+
+// SwiGLU: against the chunked kernels' 16 x 32 tiles (a workgroup each). The
+// wide kernel takes one round (12-13 us at K = 1024, 23 at 2048, 36 at 3584)
+// up to a tile of 64 x 128 per CU, theirs grow by the workgroup. us, theirs
+// against this kernel's:
+//   K = 1024: 448 tiles (3584, M = 64) 11.8 / 13.0, 512 (512, M = 512)
+//     11.5 / 12.7, 672 (3584, M = 96) 17.0 / 13.1, 2048 (16384, M = 64)
+//     19.2 / 14
+//   K = 512: 564 (3001, M = 96) 10.5 / 11.1, 1316 (M = 200) 16.8 / 11.2
+//   K = 2048: 512 (1024, M = 256) 22.7 / 23.0, 1024 (M = 512) 42.2 / 23.0
+//   K = 3584: 448 (3584, M = 64) 44 / 35.5, 672 (M = 96) 60 / 35.5
+// M <= 32 (one chunk) always stays with them.
+bool wide_swiglu_serves(int N, int K, int M) {
+  if (M <= 32 || wide_tiles(N, K, M, 64, 128) < 0) return false;
+  const long long tiles = static_cast<long long>((N + 15) / 16) * ((M + 31) / 32);
+  const long long cus = cu_count();
+  return K <= 2 * kUnit * kGroup ? 4 * tiles >= 9 * cus : 2 * tiles >= 3 * cus;
+}
+
+template <bool PACKED>
+int launch_wide_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
+                       const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,
+                       hipStream_t stream) {
+  WideArgs p = {};
+  p.w[0] = Wg;
+  p.w[1] = Wu;
+  p.s[0] = Sg;
+  p.s[1] = Su;
+  p.x = X;
+  p.y = Y;
+  p.N = N;
+  p.K = K;
+  p.M = M;
+  const bool svec = PACKED || ((K / kGroup) % 2 == 0 && aligned(Sg, 4) && aligned(Su, 4));
+  if (K <= kUnit * kGroup) {
+    if constexpr (!PACKED)
+      if (!svec) return launch_wide_t<ActBf16, 2, 2, 4, 2, PACKED, false, false, true>(p, stream);
+    return launch_wide_t<ActBf16, 2, 2, 4, 2, PACKED, true, false, true>(p, stream);
+  }
+  if constexpr (!PACKED)
+    if (!svec) return launch_wide_t<ActBf16, 2, 2, 4, 1, PACKED, false, true, true>(p, stream);
+  return launch_wide_t<ActBf16, 2, 2, 4, 1, PACKED, true, true, true>(p, stream);
+}
+
+#define W4A16_WIDE(ACT, PACKED)                                                          \
+  template int launch_wide<ACT, PACKED>(const uint8_t*, const uint16_t*, const uint16_t*, \
+                                        uint16_t*, int, int, int, hipStream_t)
+W4A16_WIDE(ActBf16, true);
+W4A16_WIDE(ActBf16, false);
+W4A16_WIDE(ActF16, true);
+W4A16_WIDE(ActF16, false);
+#undef W4A16_WIDE
+#define W4A16_WIDE_SWIGLU(PACKED)                                                          \
+  template bool wide_serves<PACKED>(int, int, int);                                       \
+  template int launch_wide_swiglu<PACKED>(const uint8_t*, const uint16_t*, const uint8_t*, \
+                                          const uint16_t*, const uint16_t*, uint16_t*, int, int, \
+                                          int, hipStream_t)
+W4A16_WIDE_SWIGLU(true);
+W4A16_WIDE_SWIGLU(false);
+#undef W4A16_WIDE_SWIGLU
+
+}  // namespace cudalm_hip

@@ -59,95 +59,6 @@ namespace {
 using namespace cudalm_hip;
 
 
-// Activation / output element type of a kernel instance. Both encode a
-// weight nibble as an exact value c + q/kUnit in the activation's 16-bit
-// format (the nibble in mantissa bits 3..6), cancel c with an MFMA against
-// -c, and scale the accumulated sum by kUnit in the epilogue.
-struct ActBf16 {
-  static constexpr uint32_t kNegOffsetPair = 0xBFC0BFC0u;  // -1.5, -1.5
-  static constexpr float kUnit = 16.0f;  // weight element = 1.5 + q / kUnit
-  template <bool ROT>
-  __device__ static u32x4_t decode(uint32_t w) { return decode_nibbles<ROT>(w); }
-  __device__ static f32x4_t mma(u32x4_t a, u32x4_t b, f32x4_t c) { return mfma16(a, b, c); }
-  __device__ static uint32_t round(float f) { return f32_to_bf16_rne(f); }
-  __device__ static float widen(uint32_t h) { return bf16_lo(h); }
-};
-
-// fp16: 1.0 = 0x3C00 with 10 mantissa bits, so q/16 sits at bit 6 and the
-// biased nibble (q + 8 = nibble ^ 8) goes to bits 6..9: 0x3C00 | 0x0200 is
-// 1.5, and the element is exactly 1.5 + q/16, the bf16 element's value. One
-// shift (one rotation from the prepacked form, which is the file dword
-// rotated left by 3) and one v_bitop3 per pair: 8 VALU ops per dword.
-// Keeping the bias at 1.5 (not 1.0625 + q/128 with the nibble at bits
-// 3..6, one op less) keeps the fp32 cancellation of the offset chain as
-// small as in bf16: the reference fixtures then stay within 0.5 fp16 ulp.
-struct ActF16 {
-  static constexpr uint32_t kNegOffsetPair = 0xBE00BE00u;  // -1.5, -1.5
-  static constexpr float kUnit = 16.0f;  // weight element = 1.5 + q / kUnit
-  template <bool ROT>
-  __device__ static u32x4_t decode(uint32_t w) {
-    u32x4_t a;
-    if constexpr (ROT) {
-      a[0] = (rotr(w, 29) & 0x03C003C0u) ^ 0x3E003E00u;
-      a[1] = (rotr(w, 1) & 0x03C003C0u) ^ 0x3E003E00u;
-      a[2] = (rotr(w, 5) & 0x03C003C0u) ^ 0x3E003E00u;
-      a[3] = (rotr(w, 9) & 0x03C003C0u) ^ 0x3E003E00u;
-    } else {
-      a[0] = ((w << 6) & 0x03C003C0u) ^ 0x3E003E00u;
-      a[1] = ((w << 2) & 0x03C003C0u) ^ 0x3E003E00u;
-      a[2] = ((w >> 2) & 0x03C003C0u) ^ 0x3E003E00u;
-      a[3] = ((w >> 6) & 0x03C003C0u) ^ 0x3E003E00u;
-    }
-    return a;
-  }
-  __device__ static f32x4_t mma(u32x4_t a, u32x4_t b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  }
-  // round to nearest even (v_cvt_f16_f32 under the default rounding mode)
-  __device__ static uint32_t round(float f) {
-    return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
-  }
-  __device__ static float widen(uint32_t h) { return half_bits_to_f32(h & 0xFFFFu); }
-};
-
-// An activation trait bound to a weight layout: decode() reads file dwords
-// (PACKED false) or prepacked, rotated dwords (PACKED true).
-template <class Act, bool PACKED>
-struct Layout : Act {
-  __device__ static u32x4_t decode(uint32_t w) { return Act::template decode<PACKED>(w); }
-};
-
-// -1.5 * (sum over the group of this lane-set's activation rows) in the
-// activation type Act.
-template <class Act>
-__device__ __forceinline__ f32x4_t group_offset_t(const u32x4_t (&xa)[4]) {
-  const u32x4_t neg = {Act::kNegOffsetPair, Act::kNegOffsetPair, Act::kNegOffsetPair,
-                       Act::kNegOffsetPair};
-  const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  f32x4_t c = Act::mma(xa[0], neg, zero);
-  c = Act::mma(xa[1], neg, c);
-  c = Act::mma(xa[2], neg, c);
-  c = Act::mma(xa[3], neg, c);
-  return c;
-}
-
-// LDS layout of staged activations. A row holds K/8 16-byte blocks plus
-// kXPad pad blocks, so rows start 2 blocks (mod 16) apart, and inside each
-// 128-column group the block of lane quarter a, step d (logical block
-// 4a + d, columns 32a + 8d ..) sits at slot 4d + a. One ds_read_b128 step
-// of a wave then reads 4 adjacent blocks from each of 16 rows: measured
-// conflict-free on gfx950 (4 LDS cycles per instruction), where unswizzled
-// rows 1 block (mod 16) apart spend half their cycles in bank conflicts.
-constexpr int kXPad = 2;
-__host__ __device__ constexpr int x_pitch(int kcl) { return (kcl >> 3) + kXPad; }
-__device__ __forceinline__ int x_slot(int c) { return (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3); }
-
-__device__ __forceinline__ void load_group_x(u32x4_t (&xa)[4], const u32x4_t* xgroup, int a) {
-#pragma unroll
-  for (int d = 0; d < 4; ++d) xa[d] = xgroup[4 * d + a];
-}
-
 // scale of group gg (0..7) from 8 packed fp16
 __device__ __forceinline__ float unit_scale(u32x4_t sv, int gg) {
   return half_bits_to_f32((sv[gg >> 1] >> (16 * (gg & 1))) & 0xFFFFu);
@@ -529,18 +440,6 @@ __device__ __forceinline__ void stream_unit(f32x4_t (&part)[CT], const StreamUni
         stream_group<NR, CT, Act, IOFF>(part, xrow, g0 + gg, cu.w[gg], corr + (g0 + gg) * 16 * CT,
                                   unit_scale(cu.s, gg), a);
   }
-}
-
-// The output of one accumulator: kUnit * total, or, when that is NaN, the
-// reference loop's sum for the output (w4a16_ref_dot: infinite and NaN
-// activations and overflow keep the reference's semantics).
-template <class Act, bool PACKED>
-__device__ __forceinline__ float out_value(float total, const uint8_t* w, const uint16_t* s, int K,
-                                           int n, const uint16_t* xrow) {
-  const float v = Act::kUnit * total;
-  if (__builtin_expect(v != v, 0))
-    return w4a16_ref_dot<PACKED, std::is_same<Act, ActF16>::value>(w, s, K, n, xrow);
-  return v;
 }
 
 // Deferred form (the streaming kernels' pipelined loops): the fast values
@@ -1536,258 +1435,6 @@ __global__ __launch_bounds__(WN * WM * 64) void w4a16_tile_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Unit GEMM kernel (prefill chunks): a k-slice of WV waves owns
-// TN = WV * RB * 16 weight rows and TM = CT * 16 activation rows. K is walked
-// one 8-group unit (1024 k) at a time: the unit's activations are staged
-// once into LDS (pair order), the slice computes the unit's offset table
-// once (waves split the chains), and every weight is decoded once, by the
-// wave that owns its rows, and feeds CT MFMA column tiles. Weights of a unit
-// are fetched up front (while the activations are staged). The per-output
-// operation sequence is the stream kernel's, so the bits are the same.
-//
-// KS > 1 k-slices split the units of the same output tile: slice s takes
-// units s, s + KS, ... with its own LDS buffers, keeps each unit partial,
-// and at the end the partials meet in LDS and are summed in unit order, so
-// the bits do not depend on KS. This serves few-tile, long-K shapes
-// (N = 1024, K = 2048 / 3584), where one slice would walk every unit alone.
-// ---------------------------------------------------------------------------
-
-constexpr int kSliceMaxUnits = 4;  // units per k-slice kept as partials (KS > 1)
-
-template <int RB, int CT, int WV, bool PACKED, bool SVEC, int KS = 1, bool IOFF = false>
-__global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
-    const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
-    const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int K, int M) {
-  constexpr int NT = WV * 64;  // threads of one k-slice
-  constexpr int TM = CT * 16;
-  constexpr int PB = x_pitch(kUnit * kGroup);  // LDS row pitch in 16-byte blocks (padded)
-  constexpr int NBLK = TM * kUnit * 16;  // 16-byte x blocks per unit
-  static_assert(NBLK % NT == 0, "staging must cover the tile exactly");
-  constexpr int BPT = NBLK / NT;  // x blocks staged per thread per unit
-  constexpr int XB = TM * PB;     // 16-byte blocks of one slice's x buffer
-  constexpr int NPART = KS == 1 ? 1 : kSliceMaxUnits;
-  extern __shared__ u32x4_t lds[];  // [KS][TM][PB] x, then [KS] offset tables
-
-  const int G = K >> 7;
-  const int U = (G + kUnit - 1) / kUnit;
-  const int ntiles = (N + kTileRows - 1) / kTileRows;
-  const int lane = threadIdx.x & 63;
-  const int slice = KS == 1 ? 0 : wave_id() / WV;
-  const int wave = wave_id() - slice * WV;  // wave within the slice
-  const int tid = static_cast<int>(threadIdx.x) - slice * NT;
-  const int i = lane & 15, a = lane >> 4;
-  const int m0 = blockIdx.y * TM;
-  const int mrows = min(TM, M - m0);
-  u32x4_t* xs = lds + slice * XB;
-  float* corr = reinterpret_cast<float*>(lds + KS * XB) + slice * (kUnit * CT * 16);
-
-  int rt[RB];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) rt[rb] = min((blockIdx.x * WV + wave) * RB + rb, ntiles - 1);
-  const bool any_ok = (blockIdx.x * WV + wave) * RB < ntiles;
-
-  // lane addresses of each owned tile at group 0
-  const uint8_t* wbase[RB];
-  const uint8_t* sbase[RB];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    if constexpr (PACKED) {
-      const uint8_t* tile = W + static_cast<size_t>(rt[rb]) * packed_tile_bytes(G);
-      wbase[rb] = tile + lane * 16;
-      sbase[rb] = tile + static_cast<size_t>(G) * 1024 + i * packed_scale_pitch(G);
-    } else {
-      const int row = min(rt[rb] * kTileRows + i, N - 1);
-      wbase[rb] = W + static_cast<size_t>(row) * (K >> 1) + a * 16;
-      sbase[rb] = reinterpret_cast<const uint8_t*>(S + static_cast<size_t>(row) * G);
-    }
-  }
-  constexpr int kStep = PACKED ? 1024 : 64;  // bytes between groups of one lane
-
-  const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  // KS == 1: the running unit sum; KS > 1: this slice's unit partials
-  f32x4_t acc[NPART][RB][CT];
-#pragma unroll
-  for (int q = 0; q < NPART; ++q)
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) acc[q][rb][ct] = zero;
-
-  const int iters = (U + KS - 1) / KS;
-  for (int it = 0; it < iters; ++it) {
-    const int u = it * KS + slice;
-    const int uc = min(u, U - 1);  // a slice past the last unit re-reads it and skips the math
-    const int g0 = uc * kUnit;
-    const int gn = u < U ? min(kUnit, G - g0) : 0;
-    // the unit's activations first: they are staged and feed the offset
-    // table before any weight is used, and loads return in issue order
-    constexpr int RS = NT / (kUnit * 16);
-    static_assert(NT % (kUnit * 16) == 0, "a thread keeps one block column");
-    const int b = tid & (kUnit * 16 - 1);  // thread tid stages block b of rows tid / 128 + q * RS
-    const int r0 = tid / (kUnit * 16);
-    u32x4_t v[BPT];
-    {
-      const uint16_t* xcol = X + static_cast<size_t>(m0) * K + min(g0 * kGroup + 8 * b, K - 8);
-#pragma unroll
-      for (int q = 0; q < BPT; ++q)
-        v[q] = *reinterpret_cast<const u32x4_t*>(
-            xcol + static_cast<size_t>(min(r0 + q * RS, mrows - 1)) * K);
-    }
-    // then this unit's weights and scales (group indices clamped to G - 1)
-    u32x4_t w[RB][kUnit];
-    uint32_t sc[RB][kUnit / 2];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-      for (int gg = 0; gg < kUnit; ++gg)
-        w[rb][gg] = *reinterpret_cast<const u32x4_t*>(
-            wbase[rb] + static_cast<size_t>(min(g0 + gg, G - 1)) * kStep);
-      if constexpr (PACKED || SVEC) {
-        const u32x4_t sv = *reinterpret_cast<const u32x4_t*>(sbase[rb] + 2 * g0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sc[rb][q] = sv[q];
-      } else {
-        const uint16_t* srow = reinterpret_cast<const uint16_t*>(sbase[rb]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          sc[rb][q] = static_cast<uint32_t>(srow[min(g0 + 2 * q, G - 1)]) |
-                      (static_cast<uint32_t>(srow[min(g0 + 2 * q + 1, G - 1)]) << 16);
-      }
-    }
-    if (it > 0) __syncthreads();  // previous unit's readers are done
-    {
-      u32x4_t* xdst = xs + r0 * PB + x_slot(b);
-#pragma unroll
-      for (int q = 0; q < BPT; ++q) xdst[q * RS * PB] = pair_order(v[q]);
-    }
-    __syncthreads();
-    // offset table of the unit: chains (group, column tile) split over waves
-    // (IOFF: each wave runs the chains of its own groups inline instead, the
-    // same operands, and the table and its barrier are skipped)
-    if constexpr (!IOFF) {
-      for (int c = wave; c < kUnit * CT; c += WV) {
-        const int gg = c / CT, ct = c - gg * CT;
-        u32x4_t xa[4];
-        load_group_x(xa, xs + (ct * 16 + i) * PB + gg * 16, a);
-        const f32x4_t o = group_offset(xa);
-        if (i == 0) *reinterpret_cast<f32x4_t*>(corr + c * 16 + 4 * a) = o;
-      }
-      __syncthreads();
-    }
-    if (!any_ok) continue;
-
-    f32x4_t part[RB][CT];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) part[rb][ct] = zero;
-    // one group: offset-seeded weight chains, then the scale fma into part
-    auto group = [&](int gg) {
-      u32x4_t xa[CT][4];
-      f32x4_t t[RB][CT];
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        load_group_x(xa[ct], xs + (ct * 16 + i) * PB + gg * 16, a);
-        const f32x4_t o = IOFF ? group_offset(xa[ct])
-                               : *reinterpret_cast<const f32x4_t*>(corr + (gg * CT + ct) * 16 + 4 * a);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) t[rb][ct] = o;
-      }
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          const u32x4_t B = decode_nibbles<PACKED>(w[rb][gg][d]);
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct) t[rb][ct] = mfma16(xa[ct][d], B, t[rb][ct]);
-        }
-      }
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const float s = half_bits_to_f32((sc[rb][gg >> 1] >> (16 * (gg & 1))) & 0xFFFFu);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            part[rb][ct][r] = __builtin_fmaf(s, t[rb][ct][r], part[rb][ct][r]);
-      }
-    };
-    if (gn == kUnit) {
-      // full unit: straight-line, so independent group chains interleave
-#pragma unroll
-      for (int gg = 0; gg < kUnit; ++gg) group(gg);
-    } else {
-#pragma unroll
-      for (int gg = 0; gg < kUnit; ++gg)
-        if (gg < gn) group(gg);
-    }
-    if constexpr (KS == 1) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) acc[0][rb][ct] = acc[0][rb][ct] + part[rb][ct];
-    } else {
-#pragma unroll
-      for (int q = 0; q < NPART; ++q)
-        if (q == it)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) acc[q][rb][ct] = part[rb][ct];
-    }
-  }
-
-  f32x4_t total[RB][CT];
-  if constexpr (KS == 1) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) total[rb][ct] = acc[0][rb][ct];
-  } else {
-    // unit partials meet in LDS (over the x buffers): slot [u][wave][rb][ct][lane]
-    __syncthreads();
-    f32x4_t* slots = reinterpret_cast<f32x4_t*>(lds);
-    if (any_ok) {
-#pragma unroll
-      for (int q = 0; q < NPART; ++q) {
-        const int u = q * KS + slice;
-        if (q < iters && u < U)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-              slots[(((u * WV + wave) * RB + rb) * CT + ct) * 64 + lane] = acc[q][rb][ct];
-      }
-    }
-    __syncthreads();
-    if (slice != 0) return;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        total[rb][ct] = zero;
-        for (int u = 0; u < U; ++u)
-          total[rb][ct] = total[rb][ct] + slots[(((u * WV + wave) * RB + rb) * CT + ct) * 64 + lane];
-      }
-  }
-  if (!any_ok) return;
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int n = ((blockIdx.x * WV + wave) * RB + rb) * kTileRows + i;
-    if (n >= N) continue;
-    uint16_t* col = Y + static_cast<size_t>(m0 + 4 * a) * N + n;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (ct * 16 + 4 * a + r < mrows)
-          col[static_cast<size_t>(ct * 16 + r) * N] = static_cast<uint16_t>(f32_to_bf16_rne(
-              out_value<ActBf16, PACKED>(total[rb][ct][r], W, S, K, n,
-                                         X + static_cast<size_t>(m0 + ct * 16 + 4 * a + r) * K)));
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Byte-wise fallback for misaligned bases (reference: int4gemv_scalar_bf16_
 // kernel, src/kernels/int4_gemv_bf16.cu:174-213): one wave per (row, m),
 // byte loads only, terms (q*s)*x in k order per lane, wave reduction.
@@ -2237,6 +1884,8 @@ template <bool PACKED>
 int launch_swiglu(const ProjTable& P, const uint16_t* X, int K, int M, hipStream_t stream) {
   const int G = K / kGroup;
   const bool svec = !PACKED && G % 8 == 0 && aligned(P.s[0], 16) && aligned(P.s[1], 16);
+  if (wide_swiglu_serves(P.n[0], K, M))
+    return launch_wide_swiglu<PACKED>(P.w[0], P.s[0], P.w[1], P.s[1], X, P.y[0], P.n[0], K, M, stream);
   const SplitPlan plan = swiglu_piece_plan(P.tile_end[0], K, M);
   if (plan.hg != 0) {
     int mc = M > 16 ? 32 : M;
@@ -2324,65 +1973,6 @@ int launch_tile(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t
   return launch_status();
 }
 
-template <int RB, int CT, int WV, bool PACKED, int KS = 1, bool IOFF = false>
-int launch_gemm_unit(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
-                     int K, int M, hipStream_t stream) {
-  constexpr int TM = CT * 16;
-  const size_t xbytes = static_cast<size_t>(TM) * x_pitch(kUnit * kGroup) * 16;
-  const size_t lds = KS * (xbytes + static_cast<size_t>(kUnit) * CT * 16 * sizeof(float));
-  const int G = K / kGroup;
-  if constexpr (KS > 1) {
-    // every slice keeps at most kSliceMaxUnits partials, and all of them
-    // must fit the x buffers they are parked in
-    const int U = (G + kUnit - 1) / kUnit;
-    if (U > KS * kSliceMaxUnits ||
-        static_cast<size_t>(U) * WV * RB * CT * 64 * 16 > KS * xbytes)
-      return launch_gemm_unit<RB, CT, WV, PACKED, 1, IOFF>(W, S, X, Y, N, K, M, stream);
-  }
-  const int ntiles = (N + kTileRows - 1) / kTileRows;
-  const int gx = (ntiles + WV * RB - 1) / (WV * RB);
-  const int gy = (M + TM - 1) / TM;
-  if (gy > 65535) return CUDALM_W4A16_ERANGE;
-  const bool svec = !PACKED && G % 8 == 0 && aligned(S, 16);
-  auto kern = svec ? w4a16_gemm_unit_kernel<RB, CT, WV, PACKED, true, KS, IOFF>
-                   : w4a16_gemm_unit_kernel<RB, CT, WV, PACKED, false, KS, IOFF>;
-  if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
-  hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(WV * KS * 64), lds, stream, W, S, X, Y, N, K, M);
-  return launch_status();
-}
-
-// Prefill chunks (M >= 33). The 32 x 32 MFMA GEMM (w4a16_gemm.hip: 32
-// activation rows x 256 weight rows per 8-wave workgroup) serves K <= 1024
-// when its workgroups fill between 3/4 and all of the CUs in one round
-// (3584x1024 and 4096x1024 at M = 512: 10.3 -> 9.6-9.9 us, 10.7 -> 9.5-10.0 us);
-// elsewhere the 16 x 16 unit GEMM is faster (one round of 32 x 256 tiles
-// leaves too many CUs idle below that, and past one round it takes two).
-// Unit GEMM tiles: 128 x 32 of 8 waves while they fill most of the CUs,
-// else 64 x 32 of 4 waves, with two k-slices of 4 waves when K spans
-// several units (1024x3584 at M = 512: 16.7 -> 14.6 us). The 4-wave tiles
-// run their offset chains inline (512x1024x512 5.8 -> 5.5 us, 1024x3584x512
-// 14.4 -> 13.8 us); inline chains cost the 8-wave tiles 0.6 us at
-// 3584x1024x512, so those keep the table.
-template <bool PACKED>
-int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
-                   int M, hipStream_t stream) {
-  const int cus = cu_count();
-  if (K == kUnit * kGroup && prefill_split_waves(N, M, cus, PACKED) != 0)
-    return launch_prefill32<PACKED>(W, S, X, Y, N, K, M, stream);
-  if (K < kUnit * kGroup) {
-    const long long wgs32 = static_cast<long long>((N + 255) / 256) * ((M + 31) / 32);
-    if (4 * wgs32 >= 3LL * cus && wgs32 <= cus)
-      return launch_prefill32<PACKED>(W, S, X, Y, N, K, M, stream);
-  }
-  const long long wgs = static_cast<long long>((N + 127) / 128) * ((M + 31) / 32);
-  // (crossover measured between 128 and 168 workgroups of 128 x 32:
-  // 2048x1024x256 5.7 vs 6.9 us, 3584x1024x192 7.4 vs 6.9 us)
-  if (5 * wgs >= 3LL * cus) return launch_gemm_unit<1, 2, 8, PACKED>(W, S, X, Y, N, K, M, stream);
-  if (K > kUnit * kGroup)
-    return launch_gemm_unit<1, 2, 4, PACKED, 2, true>(W, S, X, Y, N, K, M, stream);
-  return launch_gemm_unit<1, 2, 4, PACKED, 1, true>(W, S, X, Y, N, K, M, stream);
-}
-
 template <class Act = ActBf16>
 int launch_bytewise(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                     int K, int M, hipStream_t stream) {
@@ -2438,9 +2028,9 @@ int dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y
     case CUDALM_W4A16_VARIANT_TILE32:
       return launch_tile<1, 2, 4, 1, 8, PACKED>(W, S, X, Y, N, K, M, stream);
     case CUDALM_W4A16_VARIANT_PREFILL:
-      return launch_prefill<PACKED>(W, S, X, Y, N, K, M, stream);
+      return launch_prefill<ActBf16, PACKED>(W, S, X, Y, N, K, M, stream);
     case CUDALM_W4A16_VARIANT_PREFILL32:
-      return launch_prefill32<PACKED>(W, S, X, Y, N, K, M, stream);
+      return launch_prefill32<ActBf16, PACKED>(W, S, X, Y, N, K, M, stream);
     case CUDALM_W4A16_VARIANT_BYTEWISE:
       if (PACKED) return CUDALM_W4A16_EVARIANT;
       return launch_bytewise(W, S, X, Y, N, K, M, stream);
@@ -2449,9 +2039,11 @@ int dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y
   }
 }
 
-// fp16-activation twin: M rows in chunks that fit the stream kernels' LDS
-// (one launch when M <= 32 and x fits), the byte-wise kernel for
-// misaligned file-layout bases.
+// fp16-activation twin: the prefill kernels for M > 32, else rows in chunks
+// that fit the stream kernels' LDS (one launch when x fits), the byte-wise
+// kernel for misaligned file-layout bases. M > 32 ran 32-row chunks one after
+// the other before (us, 4096 x 1024 prepacked): M = 64 9.2 -> 4.9, 128 18.2 ->
+// 5.2, 1024 145 -> 14.7; 1024 x 3584, M = 777 337 -> 18.9.
 template <bool PACKED>
 int f16_dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                  int K, int M, bool vec_ok, hipStream_t stream) {
@@ -2459,6 +2051,7 @@ int f16_dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_
   int mc = M < 32 ? M : 32;
   while (mc > 0 && !stream_fits(K, mc, PACKED)) --mc;
   if (mc < 1) return CUDALM_W4A16_ERANGE;
+  if (M > 32 && M <= 65535 * 32) return launch_prefill<ActF16, PACKED>(W, S, X, Y, N, K, M, stream);
   for (int m0 = 0; m0 < M; m0 += mc) {
     const int rows = M - m0 < mc ? M - m0 : mc;
     const ProjTable P = single_table(W, S, Y + static_cast<size_t>(m0) * N, N);
@@ -2676,7 +2269,7 @@ int cudalm_w4a16_kernel_regs(int variant) {
       return regs_of(w4a16_stream_piece_one_kernel<true, 1, false, 1, ActBf16, 4, true, 4, false>);
     case CUDALM_W4A16_VARIANT_TILE16: return regs_of(w4a16_tile_kernel<1, 1, 4, 1, 8, true>);
     case CUDALM_W4A16_VARIANT_TILE32: return regs_of(w4a16_tile_kernel<1, 2, 4, 1, 8, true>);
-    case CUDALM_W4A16_VARIANT_PREFILL: return regs_of(w4a16_gemm_unit_kernel<1, 2, 8, true, false>);
+    case CUDALM_W4A16_VARIANT_PREFILL: return prefill_unit_regs();
     case CUDALM_W4A16_VARIANT_PREFILL32: return prefill32_regs();
     case CUDALM_W4A16_VARIANT_BYTEWISE: return regs_of(w4a16_bytewise_kernel<ActBf16>);
     case CUDALM_W4A16_VARIANT_SPLIT: return regs_of(w4a16_split_kernel<true, 1, false, 1>);

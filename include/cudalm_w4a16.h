@@ -200,7 +200,7 @@ int cudalm_w4a16_gemv_bf16_chain_noalloc(const cudalm_w4a16_stage* stages, int n
 /* fp16-activation twin of cudalm_w4a16_gemv_bf16: x and y are fp16 bit
  * patterns, y[m, n] = fp16_rne( sum_k q * f32(scale) * f32(x[m, k]) ) with
  * fp32 accumulation. Replaces int4_gemv (M == 1; include/cudalm/kernels/
- * int4_gemv.h:22-40); any M (chunks of up to 32 rows), row m bit-identical
+ * int4_gemv.h:22-40); any M, row m bit-identical
  * to the M == 1 call. Misaligned weight / x bases take a byte-wise kernel. */
 int cudalm_w4a16_gemv_f16(const uint8_t* weight, const uint16_t* scale,
                           const uint16_t* x, uint16_t* y, int N, int K, int M,
@@ -221,7 +221,8 @@ int cudalm_w4a16_gemv_f16_prepacked(const void* packed, const uint16_t* x,
  * is cudalm_silu_mul_bf16's, so y equals the reference's three-step
  * sequence gate -> up -> qwen35_silu_mul_bf16
  * (src/runtime/qwen35_deltanet.cpp:236-247) run on this library, with no
- * intermediate buffers. Any M (processed in chunks of up to 32 rows); all
+ * intermediate buffers. Any M (chunks of up to 32 rows, or the prefill GEMM
+ * for larger M); all
  * bases 16 B aligned (y: 2 B), else EALIGN. No counterpart in the
  * reference. */
 int cudalm_w4a16_swiglu_bf16(const void* gate_weight, const uint16_t* gate_scale,

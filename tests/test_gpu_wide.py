@@ -1,0 +1,117 @@
+"""The 64 x 64 wave-tile GEMM (w4a16_gemm_wide.hip): shapes its dispatch rule
+takes on a 256-CU part, at the edges of its tiles. N not a multiple of 8 (one
+output per lane in the stores), of 32 or of 256, M one row past a tile, one
+group (K = 128), odd numbers of groups, K of several 8-group units with a
+short last one, file-layout scale rows that are not 4 B aligned. Outputs must
+equal, bit for bit, those of calls of at most 32 rows, which the decode
+kernels serve (every row of a batched call equals the single-row call on it),
+for bf16 and fp16 activations, both weight layouts, non-finite activations,
+and for the SwiGLU form of the kernel; the bf16 outputs also the forced tile
+kernel's."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(51201, 128, 33), (25617, 384, 65), (3584, 1024, 897), (6152, 640, 513),
+          (5000, 1152, 700), (2056, 2176, 1473)]
+
+
+def _inputs(dev, N, K, M, dtype, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    w = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device=dev, generator=g)
+    s = (torch.rand(N, K // 128, device=dev, generator=g) * 0.01 + 0.001).to(torch.float16)
+    return w, s, torch.randn(M, K, device=dev, generator=g).to(dtype)
+
+
+def _bits(t):
+    return t.contiguous().view(torch.int16)
+
+
+def _same(a, b, label):
+    # equal bits, except that any NaN equals any other
+    diff = (_bits(a) != _bits(b)) & ~(a.isnan() & b.isnan())
+    torch.cuda.synchronize()
+    assert int(diff.sum()) == 0, (label, int(diff.sum()), a.shape)
+
+
+def _by_chunks(call, x, N):
+    y = torch.empty(x.shape[0], N, dtype=x.dtype, device=x.device)
+    for m0 in range(0, x.shape[0], 32):
+        xc = x[m0:m0 + 32].contiguous()
+        call(xc, xc.shape[0], y[m0:m0 + 32])
+    return y
+
+
+@pytest.mark.parametrize("N,K,M", SHAPES)
+@pytest.mark.parametrize("f16", [False, True])
+def test_wide_equals_decode_kernels(w4, dev, N, K, M, f16):
+    dtype = torch.float16 if f16 else torch.bfloat16
+    w, s, x = _inputs(dev, N, K, M, dtype, 0x71DE + N + K + M)
+    # scales 2 bytes past a 4-byte boundary
+    buf = torch.empty(s.numel() + 1, dtype=torch.float16, device=dev)
+    s2 = buf[1:].view_as(s)
+    s2.copy_(s)
+    assert s2.data_ptr() % 4 == 2
+    p = w4.repack(w, s, N, K)
+    file_call = w4.gemv_f16 if f16 else w4.gemv
+    packed_call = w4.gemv_f16_prepacked if f16 else w4.gemv_prepacked
+    for bad in (False, True):
+        if bad:
+            x[M // 2, K // 3] = float("inf")
+            x[M - 1, 1] = float("nan")
+            x[0, K - 1] = -float("inf")
+        ref = _by_chunks(lambda xc, m, yc: packed_call(p, xc, N, K, m, y=yc), x, N)
+        for label, call in (("prepacked", lambda y: packed_call(p, x, N, K, M, y=y)),
+                            ("file", lambda y: file_call(w, s, x, N, K, M, y=y)),
+                            ("scales", lambda y: file_call(w, s2, x, N, K, M, y=y))):
+            y = torch.empty(M, N, dtype=dtype, device=dev)
+            call(y)
+            _same(y, ref, (label, bad))
+        if not f16:
+            y = torch.empty(M, N, dtype=dtype, device=dev)
+            w4.gemv(w, s, x, N, K, M, y=y, variant="tile32")
+            _same(y, ref, ("tile32", bad))
+    # an output base off 16 bytes
+    yb = torch.empty(M * N + 1, dtype=dtype, device=dev)
+    y = yb[1:].view(M, N)
+    packed_call(p, x, N, K, M, y=y)
+    _same(y, ref, "output base")
+
+
+@pytest.mark.parametrize("N,K,M", [(3584, 1024, 100), (3584, 1024, 833), (8200, 384, 70),
+                                   (16385, 128, 40), (2048, 2176, 300), (3000, 3584, 65)])
+def test_wide_swiglu_equals_chunks(w4, dev, N, K, M):
+    gw, gs, x = _inputs(dev, N, K, M, torch.bfloat16, 0x51F + N + M)
+    uw, us, _ = _inputs(dev, N, K, 1, torch.bfloat16, 0x520 + K)
+    gp, up = w4.repack(gw, gs, N, K), w4.repack(uw, us, N, K)
+    for bad in (False, True):
+        if bad:
+            x[M // 2, K // 3] = float("inf")
+            x[M - 1, 1] = float("nan")
+        ref = _by_chunks(lambda xc, m, yc: w4.swiglu(gp, None, up, None, xc, N, K, m, y=yc,
+                                                     prepacked=True), x, N)
+        y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        w4.swiglu(gp, None, up, None, x, N, K, M, y=y, prepacked=True)
+        _same(y, ref, ("prepacked", bad))
+        y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        w4.swiglu(gw, gs, uw, us, x, N, K, M, y=y)
+        _same(y, ref, ("file", bad))
+
+
+@pytest.mark.parametrize("N,K,M", [(4096, 1024, 33), (512, 1024, 128), (1000, 640, 70),
+                                   (37, 3584, 65), (3584, 512, 512), (6144, 1024, 512)])
+def test_f16_prefill_equals_decode_kernels(w4, dev, N, K, M):
+    # the smaller-tiled prefill kernels on fp16 activations (each of the split
+    # kernel's widths, the 32 x 32 kernel and the unit GEMM's forms)
+    w, s, x = _inputs(dev, N, K, M, torch.float16, 0xF16 + N + K + M)
+    p = w4.repack(w, s, N, K)
+    x[M // 2, 3] = float("inf")
+    ref = _by_chunks(lambda xc, m, yc: w4.gemv_f16_prepacked(p, xc, N, K, m, y=yc), x, N)
+    y = torch.empty(M, N, dtype=torch.float16, device=dev)
+    w4.gemv_f16_prepacked(p, x, N, K, M, y=y)
+    _same(y, ref, "prepacked")
+    y = torch.empty(M, N, dtype=torch.float16, device=dev)
+    w4.gemv_f16(w, s, x, N, K, M, y=y)
+    _same(y, ref, "file")
