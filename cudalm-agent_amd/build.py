@@ -17,7 +17,7 @@ REPO = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB = os.path.join(PKG_DIR, "cudalm_w4a16", "libcudalm_w4a16.so")
 SOURCES = ["w4a16_kernels.hip", "w4a16_chain.hip", "w4a16_gemm.hip", "w4a16_gemm_wide.hip",
-           "bf16_gemv_kernels.hip", "w4a16_host.hip", "cudalm_v2_reader.cpp"]
+           "bf16_gemv_kernels.hip", "bf16_gemm.hip", "w4a16_host.hip", "cudalm_v2_reader.cpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -7,7 +7,8 @@
 //   W bf16 [N, K], x bf16 [M, K], y bf16 [M, N], all row-major.
 //
 // The weight is read exactly once per launch (for M <= 32 activation rows;
-// larger M is split into row chunks that each stream it). bf16 x bf16
+// larger M takes the GEMM of bf16_gemm.hip, or, where the matrix is small,
+// row chunks that each stream it). bf16 x bf16
 // products are exact in fp32, so the matrix cores compute the contraction
 // directly: v_mfma_f32_16x16x32_bf16 with activations as the A operand and
 // a 16-row weight tile as the B operand. Lane l = 16a + i of MFMA step j in
@@ -28,6 +29,7 @@
 #include <stdint.h>
 #include <stdlib.h>
 
+#include "bf16_gemm.h"
 #include "cudalm_bf16_gemv.h"
 #include "hip_common.h"
 
@@ -270,11 +272,30 @@ int launch_stream_ct(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, i
   return launch_status();
 }
 
+// M > 32: the GEMM (bf16_gemm.hip), which reads the weights once (twice for M
+// in 129 .. 256, from L2 the second time), against chunks of mc rows that each
+// stream them. The chunks' workgroups (64 weight rows each) cost little while
+// they fill the CUs once; the GEMM takes one round of 10 us (K = 1024) to 26 us
+// (K = 3072), 14 to 35 with 128-row tiles. Chunks / GEMM, us, by workgroups on
+// 256 CUs: K = 1024: 256 (8192, M = 64) 10.1 / 10.6, 512 (16384, M = 64) 11.9 /
+// 11.1, (4096, M = 256) 11.7 / 14.0, 1024 (8192, M = 256) 22.9 / 15.0; K = 512:
+// 512 7.2 / 7.0, 1024 11.9 / 9.4; tile-major copy, K = 1024: 512 (16384, M =
+// 64) 9.9 / 11.3, 768 (M = 96) 18.1 / 14.9; K = 3072 (24-row chunks, one workgroup per
+// CU): 176 (1024, M = 256) 22.6 / 34.7, 384 (8192, M = 64) 39.4 / 26.3.
+bool prefer_gemm(int N, int K, int M, int mc, bool packed) {
+  if (M <= 32 || !bf16_gemm_fits(N, M)) return false;
+  const long long wgs = static_cast<long long>((N + 63) / 64) * ((M + mc - 1) / mc);
+  const long long cus = cu_count();
+  if (K > 1024) return wgs > cus;
+  return wgs >= (M <= 64 && !packed ? 2 : 3) * cus;
+}
+
 template <bool PACKED = false>
 int launch_stream(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int K, int M,
                   hipStream_t stream) {
   const int mc = stream_rows_per_chunk(K, M);
   if (mc < 1) return CUDALM_W4A16_EVARIANT;
+  if (prefer_gemm(N, K, M, mc, PACKED)) return launch_bf16_gemm<PACKED>(W, X, Y, N, K, M, stream);
   if (mc > 16) return launch_stream_ct<2, PACKED>(W, X, Y, N, K, M, mc, stream);
   return launch_stream_ct<1, PACKED>(W, X, Y, N, K, M, mc, stream);
 }

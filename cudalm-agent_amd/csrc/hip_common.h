@@ -49,11 +49,62 @@ __device__ __forceinline__ uint32_t f32_to_bf16_rne(float f) {
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
+// The same on two values, one dword (lo in bits 0..15).
+__device__ __forceinline__ uint32_t f32_to_bf16_rne2(float lo, float hi) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2_t{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
+}
+
 // D = A (16 rows x 32 k) * B (32 k x 16 cols) + C, bf16 in, fp32 accumulate.
 // Lane l = 16a + i: A row i / B column i, k = 8a .. 8a+7; D rows 4a..4a+3 of column i.
 __device__ __forceinline__ f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// Output tile of one wave on its way to memory through LDS: rows of BNW
+// 16-bit elements, kOutPad more per row so that rows spread over the banks.
+constexpr int kOutPad = 8;
+
+// Two vertically adjacent outputs of column j (rows r and r + 1, one dword)
+// per lane: neighbouring lanes swap theirs so that the even lane writes row
+// r, the odd one row r + 1, both columns of the pair (16-bit LDS writes cost
+// as many LDS cycles each). `pair` is row (j & 1), column (j & ~1) of the
+// tile; dst selects the rows and columns from there.
+__device__ __forceinline__ void put_row_pair(uint16_t* dst, uint32_t own, int j) {
+  const uint32_t other = static_cast<uint32_t>(
+      __builtin_amdgcn_mov_dpp(static_cast<int>(own), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+  // v_perm_b32 over (other:own): even own.lo | other.lo << 16, odd other.hi | own.hi << 16
+  *reinterpret_cast<uint32_t*>(dst) =
+      __builtin_amdgcn_perm(other, own, (j & 1) ? 0x03020706u : 0x05040100u);
+}
+
+// Rows [0, mrows) x columns [0, ncols) of the tile `ot` to yt (row pitch N
+// elements): 16 bytes per lane where every row of y starts 16 B aligned (whole8),
+// else one output per lane.
+template <int BM, int BNW>
+__device__ __forceinline__ void store_rows(uint16_t* yt, int N, const uint16_t* ot, int mrows,
+                                           int ncols, int lane, bool whole8) {
+  constexpr int kPitch = BNW + kOutPad;
+  if (whole8) {
+    constexpr int LPR = BNW / 8;   // lanes per row
+    constexpr int RPI = 64 / LPR;  // rows per store
+    const int c = 8 * (lane % LPR), r0 = lane / LPR;
+    if (c < ncols) {
+#pragma unroll
+      for (int r = 0; r < BM; r += RPI)
+        if (r + r0 < mrows)
+          *reinterpret_cast<u32x4_t*>(yt + static_cast<size_t>(r + r0) * N + c) =
+              *reinterpret_cast<const u32x4_t*>(ot + (r + r0) * kPitch + c);
+    }
+  } else {
+    constexpr int CPI = BNW < 64 ? BNW : 64;
+    const int c0 = lane % CPI, r0 = lane / CPI;
+    for (int r = r0; r < mrows; r += 64 / CPI)
+#pragma unroll
+      for (int c = c0; c < BNW; c += 64)
+        if (c < ncols) yt[static_cast<size_t>(r) * N + c] = ot[r * kPitch + c];
+  }
 }
 
 inline bool aligned(const void* p, uintptr_t a) {

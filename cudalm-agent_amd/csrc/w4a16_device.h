@@ -93,11 +93,8 @@ struct ActBf16 {
   __device__ static u32x4_t decode(uint32_t w) { return decode_nibbles<ROT>(w); }
   __device__ static f32x4_t mma(u32x4_t a, u32x4_t b, f32x4_t c) { return mfma16(a, b, c); }
   __device__ static uint32_t round(float f) { return f32_to_bf16_rne(f); }
-  // two roundings in one dword (lo in bits 0..15): one v_cvt_pk_bf16_f32
-  __device__ static uint32_t round2(float lo, float hi) {
-    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, bf16x2_t{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
-  }
+  // two roundings in one dword (lo in bits 0..15)
+  __device__ static uint32_t round2(float lo, float hi) { return f32_to_bf16_rne2(lo, hi); }
   __device__ static float widen(uint32_t h) { return bf16_lo(h); }
 };
 

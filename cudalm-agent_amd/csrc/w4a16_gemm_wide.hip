@@ -373,10 +373,9 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
   __syncthreads();
   if (!wave_ok) return;
   constexpr bool F16 = std::is_same<Act, ActF16>::value;
-  constexpr int kOutPitch = BNW + 8;  // 16-bit elements per LDS output row (padded)
+  constexpr int kOutPitch = BNW + kOutPad;  // 16-bit elements per LDS output row
   static_assert(static_cast<size_t>(WV) * BM * kOutPitch * 2 <= wide_lds_bytes<MT>(), "fits");
   uint16_t* const ot = reinterpret_cast<uint16_t*>(lds) + wave * BM * kOutPitch;
-  const uint32_t psel = (j & 1) ? 0x03020706u : 0x05040100u;  // v_perm_b32 over (other:own)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     // one unit: total = 0 + part; kUnit * total in one exact fma
@@ -390,11 +389,7 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
 #pragma unroll
       for (int r = 0; r < 16; r += 2) bad |= __builtin_isunordered(v[nt][r], v[nt][r + 1]);
     }
-    // Rows r and r + 1 of column j are one dword; neighbouring lanes swap
-    // theirs so that the even lane writes row r, the odd one row r + 1, both
-    // columns of the pair (16-bit LDS writes cost as many LDS cycles each).
-    uint16_t* const pair =
-        ot + (mt * 32 + 4 * h + (j & 1)) * kOutPitch + (j & ~1);
+    uint16_t* const pair = ot + (mt * 32 + 4 * h + (j & 1)) * kOutPitch + (j & ~1);
 #pragma unroll
     for (int r = 0; r < 16; r += 2)
 #pragma unroll
@@ -405,11 +400,7 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
                 silu_mul_bits(f32_to_bf16_rne(v[0][r + 1]), f32_to_bf16_rne(v[1][r + 1])) << 16;
         else
           own = Act::round2(v[nt][r], v[nt][r + 1]);
-        const uint32_t other = static_cast<uint32_t>(
-            __builtin_amdgcn_mov_dpp(static_cast<int>(own), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-        // even: own.lo | other.lo << 16; odd: other.hi | own.hi << 16
-        *reinterpret_cast<uint32_t*>(pair + (8 * (r >> 2) + (r & 3)) * kOutPitch + 32 * nt) =
-            __builtin_amdgcn_perm(other, own, psel);
+        put_row_pair(pair + (8 * (r >> 2) + (r & 3)) * kOutPitch + 32 * nt, own, j);
       }
     if (__builtin_expect(bad, 0)) {
       // outputs whose fast sum is NaN: the reference loop's value instead
@@ -449,29 +440,8 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
     }
   }
   wave_lds_sync();
-  // rows out: 16 bytes per lane where every row of y starts 16 B aligned,
-  // else one output per lane
-  uint16_t* const yt = p.y + static_cast<size_t>(m0) * N + nbase;
-  const int ncols = min(BNW, N - nbase);
-  if ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0) {
-    constexpr int LPR = BNW / 8;   // lanes per row
-    constexpr int RPI = 64 / LPR;  // rows per store
-    const int c = 8 * (lane % LPR), r0 = lane / LPR;
-    if (c < ncols) {
-#pragma unroll
-      for (int r = 0; r < BM; r += RPI)
-        if (r + r0 < mrows)
-          *reinterpret_cast<u32x4_t*>(yt + static_cast<size_t>(r + r0) * N + c) =
-              *reinterpret_cast<const u32x4_t*>(ot + (r + r0) * kOutPitch + c);
-    }
-  } else {
-    constexpr int RPI = 64 / (BNW < 64 ? BNW : 64);
-    const int c0 = lane % (BNW < 64 ? BNW : 64), r0 = lane / (BNW < 64 ? BNW : 64);
-    for (int r = r0; r < mrows; r += RPI)
-#pragma unroll
-      for (int c = c0; c < BNW; c += 64)
-        if (c < ncols) yt[static_cast<size_t>(r) * N + c] = ot[r * kOutPitch + c];
-  }
+  store_rows<BM, BNW>(p.y + static_cast<size_t>(m0) * N + nbase, N, ot, mrows, min(BNW, N - nbase),
+                      lane, (N & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
 }
 
 template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU>
