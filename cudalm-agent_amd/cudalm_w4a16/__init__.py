@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libcudalm_w4a16.so")
@@ -177,13 +178,26 @@ def _ptr(t) -> int | None:
     return t.data_ptr()
 
 
-def _stream(stream) -> int | None:
-    import torch  # noqa: F401  (torch owns the streams)
+def _current_stream() -> int:
+    """Raw handle of torch's current stream on the current device, through the
+    accessors torch's own generated launchers use: 0.2 us, where building the
+    Stream object of torch.cuda.current_stream() takes 2.8 us, as long as a
+    decode projection runs (3584x1024, M = 1: 7.6 -> 4.7 us per call)."""
+    import torch
 
+    if torch.cuda.is_initialized():
+        try:
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:  # a torch without these accessors
+            pass
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _stream(stream) -> int | None:
+    if stream is None:
+        return _current_stream()
     if isinstance(stream, int):
         return stream  # a raw hipStream_t (0 = the null stream)
-    if stream is None:
-        stream = torch.cuda.current_stream()
     return stream.cuda_stream
 
 
@@ -308,11 +322,14 @@ def gemv_multi(weights, scales, x, Ns, K: int, M: int = 1, ys=None, prepacked: b
 
     if ys is None:
         ys = [torch.empty((M, n), dtype=torch.bfloat16, device=x.device) for n in Ns]
-    items = [(_ptr(w), None if (prepacked or s is None) else _ptr(s), _ptr(y), n)
-             for w, s, y, n in zip(weights, scales if scales is not None else [None] * len(Ns), ys, Ns)]
-    arr = proj_array(items)
-    rc = _lib.cudalm_w4a16_gemv_bf16_multi(ctypes.cast(arr, ctypes.c_void_p), len(items), _ptr(x),
-                                           K, M, int(prepacked), _stream(stream))
+    # the array of struct cudalm_w4a16_proj as bytes: one pack instead of a
+    # ctypes attribute store per field
+    fields = []
+    for w, s, y, n in zip(weights, scales if scales is not None else [None] * len(Ns), ys, Ns):
+        fields += (_ptr(w) or 0, 0 if (prepacked or s is None) else _ptr(s), _ptr(y) or 0, n)
+    count = len(fields) // 4
+    rc = _lib.cudalm_w4a16_gemv_bf16_multi(struct.pack("PPPi4x" * count, *fields), count, _ptr(x), K,
+                                           M, int(prepacked), _stream(stream))
     _check(rc, "cudalm_w4a16_gemv_bf16_multi")
     return ys
 
