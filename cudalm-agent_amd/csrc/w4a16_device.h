@@ -287,6 +287,13 @@ template <class Act, bool PACKED>
 int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
                 int M, hipStream_t stream);
 
+// Its form with k-slices of one unit each, for few tiles of 2048 < K <= 4096.
+template <bool PACKED>
+bool wide_slices_serve(const uint16_t* S, int N, int K, int M);
+template <class Act, bool PACKED>
+int launch_wide_slices(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
+                       int K, int M, hipStream_t stream);
+
 // The same kernel over gate and up, storing silu(gate) * up.
 bool wide_swiglu_serves(int N, int K, int M);
 template <bool PACKED>

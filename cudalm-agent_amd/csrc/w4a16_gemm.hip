@@ -896,6 +896,8 @@ int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint1
                    int M, hipStream_t stream) {
   const int cus = cu_count();
   if (wide_serves<PACKED>(N, K, M)) return launch_wide<Act, PACKED>(W, S, X, Y, N, K, M, stream);
+  if (wide_slices_serve<PACKED>(S, N, K, M))
+    return launch_wide_slices<Act, PACKED>(W, S, X, Y, N, K, M, stream);
   if (K == kUnit * kGroup && prefill_split_waves(N, M, cus, PACKED) != 0)
     return launch_prefill32<Act, PACKED>(W, S, X, Y, N, K, M, stream);
   if (K < kUnit * kGroup) {

@@ -41,7 +41,9 @@
 // also runs their offset chains. Weights and scales are loaded one group
 // ahead into registers. The operands of a 16-k step are read and decoded
 // during the step before, pinned there by scheduling barriers: left alone
-// the compiler reads them just in time.
+// the compiler reads them just in time. With KS k-slices a workgroup has KS
+// such wave sets, each on one 8-group unit of the same outputs with buffers
+// of its own; the unit partials meet in LDS and are summed in unit order.
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -85,21 +87,27 @@ struct WideArgs {
 };
 
 // SVEC: 4-byte aligned scale pairs (prepacked, or G even and S 4 B aligned)
-template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU>
-__global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs p) {
+template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU,
+          int KS = 1>
+__global__ __launch_bounds__(WV * KS * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs p) {
   static_assert(!GLU || NT == 2, "a wave holds a gate and an up tile");
+  static_assert(KS == 1 || (!GLU && !MULTI), "a k-slice is one unit");
   constexpr int BM = 32 * MT;
   constexpr int BNW = GLU ? 32 : 32 * NT;  // output columns per wave
   constexpr int NS = BM / 16;              // 16-row staging slices
   constexpr int SPW = (NS + WV - 1) / WV;  // slices per wave
   extern __shared__ u32x4_t lds[];
   constexpr int XB = BM * kWidePitch;  // 16-byte blocks of one group's x
-  float* const ob = reinterpret_cast<float*>(lds + 4 * XB);
+  const int slice = KS == 1 ? 0 : wave_id() / WV;
+  u32x4_t* const xs = lds + slice * (wide_lds_bytes<MT>() / 16);
+  float* const ob = reinterpret_cast<float*>(xs + 4 * XB);
 
   const int K = p.K, N = p.N;
   const int G = K >> 7;
+  // this slice's groups: [gb, ge), all of them or one 8-group unit
+  const int gb = slice * kUnit, ge = KS == 1 ? G : min(G, gb + kUnit);
   const int lane = threadIdx.x & 63;
-  const int wave = wave_id();
+  const int wave = wave_id() - slice * WV;
   const int j = lane & 31, h = lane >> 5;
   const int i16 = lane & 15, a16 = lane >> 4;
 
@@ -305,13 +313,13 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
   };
   // prologue: the first two groups of x, then the first weights
   {
-    load_x(0);
+    load_x(min(gb, G - 1));
     u32x4_t x0[SPW][4];
 #pragma unroll
     for (int sl = 0; sl < SPW; ++sl)
 #pragma unroll
       for (int q = 0; q < 4; ++q) x0[sl][q] = xr[sl][q];
-    load_x(min(1, G - 1));
+    load_x(min(gb + 1, G - 1));
     u32x4_t x1[SPW][4];
 #pragma unroll
     for (int sl = 0; sl < SPW; ++sl)
@@ -320,57 +328,111 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
         x1[sl][q] = xr[sl][q];
         xr[sl][q] = x0[sl][q];
       }
-    load_w(w0, 0);
-    load_s(sc, 0);
-    stage_write(lds);
+    load_w(w0, min(gb, G - 1));
+    load_s(sc, min(gb, (G - 1) & ~1));
+    stage_write(xs);
 #pragma unroll
     for (int sl = 0; sl < SPW; ++sl)
 #pragma unroll
       for (int q = 0; q < 4; ++q) xr[sl][q] = x1[sl][q];
-    stage_write(lds + XB);
-    load_x(min(2, G - 1));
+    stage_write(xs + XB);
+    load_x(min(gb + 2, G - 1));
+    // both groups' offset chains side by side, all their reads ahead
+    wave_lds_sync();
+    u32x4_t xq[2][SPW][4];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int sl = 0; sl < SPW; ++sl)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          xq[q][sl][d] = xs[q * XB + (16 * min(wave + sl * WV, NS - 1) + i16) * kWidePitch + 4 * a16 + d];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        stage_read(lds + q * XB, d);
-        stage_chain(d);
-      }
+      for (int sl = 0; sl < SPW; ++sl) oc[sl] = group_offset_t<Act>(xq[q][sl]);
       stage_table(ob + q * BM);
     }
   }
   __syncthreads();
-  int g = 0, cur = 0;
-  for (; g + 1 < G; g += 2, cur ^= 2) {
+  int g = gb, cur = 0;
+  // (k-slices all walk whole units: they share the barriers)
+  for (; KS == 1 ? g + 1 < G : g < gb + kUnit; g += 2, cur ^= 2) {
     // groups g and g + 1 from one buffer pair, g + 2 and g + 3 staged into
     // the other meanwhile
     const int nxt = cur ^ 2;
-    group(lds + cur * XB, ob + cur * BM, w0, sc, 0, [&](int s) {
-      if (s == 0) stage_write(lds + nxt * XB);
+    const auto even = [&] { group(xs + cur * XB, ob + cur * BM, w0, sc, 0, [&](int s) {
+      if (s == 0) stage_write(xs + nxt * XB);
       if (s == 1) load_x(min(g + 3, G - 1));
-      if (s == 1) load_w(w1, g + 1);
+      if (s == 1) load_w(w1, KS == 1 ? g + 1 : min(g + 1, G - 1));
       if (s == 1) load_s(scn, min(g + 2, (G - 1) & ~1));
       if (s >= 3 && s < 7) stage_chain(s - 3);
-      if (s >= 2 && s < 6) stage_read(lds + nxt * XB, s - 2);
+      if (s >= 2 && s < 6) stage_read(xs + nxt * XB, s - 2);
       if (s == 7) stage_table(ob + nxt * BM);
-    }, [] {});
-    group(lds + cur * XB + XB, ob + cur * BM + BM, w1, sc, 1, [&](int s) {
-      if (s == 0) stage_write(lds + nxt * XB + XB);
+    }, [] {}); };
+    const auto odd = [&] { group(xs + cur * XB + XB, ob + cur * BM + BM, w1, sc, 1, [&](int s) {
+      if (s == 0) stage_write(xs + nxt * XB + XB);
       if (s == 1) load_x(min(g + 4, G - 1));
       if (s == 1) load_w(w0, min(g + 2, G - 1));
       if (s >= 3 && s < 7) stage_chain(s - 3);
-      if (s >= 2 && s < 6) stage_read(lds + nxt * XB + XB, s - 2);
+      if (s >= 2 && s < 6) stage_read(xs + nxt * XB + XB, s - 2);
       if (s == 7) stage_table(ob + nxt * BM + BM);
-    }, [] { __syncthreads(); });
+    }, [] { if (KS == 1) __syncthreads(); }); };
+    if constexpr (KS == 1) {
+      even();
+      odd();
+    } else {
+      if (g < ge) even();
+      if (g + 1 < ge) odd();
+      __syncthreads();
+    }
     if (MULTI && (g & 7) == 6) fold();
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) sc[nt] = scn[nt];
   }
-  if (g < G) group(lds + cur * XB, ob + cur * BM, w0, sc, 0, [](int) {}, [] {});
+  if (KS == 1 && g < G) group(xs + cur * XB, ob + cur * BM, w0, sc, 0, [](int) {}, [] {});
   if (MULTI && (G & 7) != 0) fold();
   // every wave is done with the staged x; from here on each wave has its own
   // part of the LDS
   __syncthreads();
+  if constexpr (KS > 1) {
+    // unit partials meet in LDS and slice 0 sums them in unit order
+    f32x4_t* const slots = reinterpret_cast<f32x4_t*>(lds) + (wave * MT * NT * 4) * 64 + lane;
+    constexpr int SLICE = WV * MT * NT * 4 * 64;  // f32x4 slots per slice
+    static_assert(static_cast<size_t>(KS - 1) * SLICE * 16 <= KS * wide_lds_bytes<MT>(), "fits");
+    if (slice > 0) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            slots[(slice - 1) * SLICE + ((mt * NT + nt) * 4 + q) * 64] =
+                f32x4_t{part[mt][nt][4 * q], part[mt][nt][4 * q + 1], part[mt][nt][4 * q + 2],
+                        part[mt][nt][4 * q + 3]};
+    }
+    __syncthreads();
+    if (slice == 0) {
+      const int U = (G + kUnit - 1) / kUnit;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) part[mt][nt] = zero16 + part[mt][nt];
+      for (int u = 1; u < U; ++u)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const f32x4_t o = slots[(u - 1) * SLICE + ((mt * NT + nt) * 4 + q) * 64];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) part[mt][nt][4 * q + r] = part[mt][nt][4 * q + r] + o[r];
+            }
+    }
+    __syncthreads();
+    if (slice != 0) return;
+  }
   if (!wave_ok) return;
   constexpr bool F16 = std::is_same<Act, ActF16>::value;
   constexpr int kOutPitch = BNW + kOutPad;  // 16-bit elements per LDS output row
@@ -444,17 +506,23 @@ __global__ __launch_bounds__(WV * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs 
                       lane, (N & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
 }
 
-template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU>
+template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU,
+          int KS = 1>
 int launch_wide_t(WideArgs p, hipStream_t stream) {
   constexpr int BN = WV * (GLU ? 32 : 32 * NT);
   p.tiles_m = (p.M + 32 * MT - 1) / (32 * MT);
   p.tiles_n = (p.N + BN - 1) / BN;
-  auto kern = w4a16_gemm_wide_kernel<Act, MT, NT, WV, OCC, PACKED, SVEC, MULTI, GLU>;
-  const size_t lds = wide_lds_bytes<MT>();
+  auto kern = w4a16_gemm_wide_kernel<Act, MT, NT, WV, OCC, PACKED, SVEC, MULTI, GLU, KS>;
+  const size_t lds = KS * wide_lds_bytes<MT>();
   if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
   const int grid = 8 * ((p.tiles_m * p.tiles_n + 7) / 8);  // an equal run of tiles per XCD
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(WV * 64), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(WV * KS * 64), lds, stream, p);
   return launch_status();
+}
+
+WideArgs wide_args(const uint8_t* W0, const uint16_t* S0, const uint8_t* W1, const uint16_t* S1,
+                   const uint16_t* X, uint16_t* Y, int N, int K, int M) {
+  return WideArgs{{W0, W1}, {S0, S1}, X, Y, N, K, M, 0, 0};
 }
 
 // Tiles of BM x BN outputs, -1 beyond the kernel's index ranges (32-bit tile
@@ -485,14 +553,7 @@ bool wide_serves(int N, int K, int M) {
 template <class Act, bool PACKED>
 int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
                 int M, hipStream_t stream) {
-  WideArgs p = {};
-  p.w[0] = p.w[1] = W;
-  p.s[0] = p.s[1] = S;
-  p.x = X;
-  p.y = Y;
-  p.N = N;
-  p.K = K;
-  p.M = M;
+  const WideArgs p = wide_args(W, S, W, S, X, Y, N, K, M);
   const bool svec = PACKED || ((K / kGroup) % 2 == 0 && aligned(S, 4));
   if (K <= kUnit * kGroup) {
     if constexpr (!PACKED)
@@ -502,6 +563,36 @@ int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t
   if constexpr (!PACKED)
     if (!svec) return launch_wide_t<Act, 2, 1, 4, 2, PACKED, false, true, false>(p, stream);
   return launch_wide_t<Act, 2, 1, 4, 2, PACKED, true, true, false>(p, stream);
+}
+
+// Few tiles of long K (a down projection): four k-slices of one unit each per
+// 32 x 128 tile, 16 waves, where the unit GEMM's 64 x 32 tiles no longer fill
+// one round and its 128 x 32 tiles, one slice of 8 waves, walk every unit
+// alone. 1024 x 3584 prepacked / file layout, unit GEMM first: M = 777 18.7 ->
+// 15.5 / 22.4 -> 18.4 us, M = 1000 20.0 -> 16.2 / 23.4 -> 18.7; 2048 x 4096, M =
+// 500 19.0 -> 17.8 / 21.1 -> 22.0, so the file layout takes it only where the
+// unit GEMM cannot load a unit's scales at once (K / 128 not a multiple of 8).
+// Below one round of 64 x 32 tiles (M = 512: 12.9 against 14.7 us) and at
+// short K the unit GEMM is faster (K = 2048, two slices, M = 777 9.9 against
+// 10.6 us; prepacked 4096 x 2304, M = 256 11.1 against 11.5, file layout 14.7
+// against 12.6). What
+// bounds the slices is VALU: at 32 rows a decoded dword feeds one MFMA.
+template <bool PACKED>
+bool wide_slices_serve(const uint16_t* S, int N, int K, int M) {
+  if (K <= (PACKED ? 20 * kGroup : 2 * kUnit * kGroup) || K > 4 * kUnit * kGroup) return false;
+  if (!PACKED && (K / kGroup) % 8 == 0 && aligned(S, 16)) return false;
+  const long long rows = (M + 31) / 32, cus = cu_count();
+  return rows * ((N + 63) / 64) > cus && rows * ((N + 127) / 128) <= cus;
+}
+
+template <class Act, bool PACKED>
+int launch_wide_slices(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
+                       int K, int M, hipStream_t stream) {
+  const WideArgs p = wide_args(W, S, W, S, X, Y, N, K, M);
+  if constexpr (!PACKED)
+    if ((K / kGroup) % 2 != 0 || !aligned(S, 4))
+      return launch_wide_t<Act, 1, 1, 4, 1, PACKED, false, false, false, 4>(p, stream);
+  return launch_wide_t<Act, 1, 1, 4, 1, PACKED, true, false, false, 4>(p, stream);
 }
 
 // SwiGLU: against the chunked kernels' 16 x 32 tiles (a workgroup each). The
@@ -526,16 +617,7 @@ template <bool PACKED>
 int launch_wide_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
                        const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,
                        hipStream_t stream) {
-  WideArgs p = {};
-  p.w[0] = Wg;
-  p.w[1] = Wu;
-  p.s[0] = Sg;
-  p.s[1] = Su;
-  p.x = X;
-  p.y = Y;
-  p.N = N;
-  p.K = K;
-  p.M = M;
+  const WideArgs p = wide_args(Wg, Sg, Wu, Su, X, Y, N, K, M);
   const bool svec = PACKED || ((K / kGroup) % 2 == 0 && aligned(Sg, 4) && aligned(Su, 4));
   if (K <= kUnit * kGroup) {
     if constexpr (!PACKED)
@@ -548,6 +630,9 @@ int launch_wide_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
 }
 
 #define W4A16_WIDE(ACT, PACKED)                                                          \
+  template int launch_wide_slices<ACT, PACKED>(const uint8_t*, const uint16_t*,          \
+                                               const uint16_t*, uint16_t*, int, int, int, \
+                                               hipStream_t);                             \
   template int launch_wide<ACT, PACKED>(const uint8_t*, const uint16_t*, const uint16_t*, \
                                         uint16_t*, int, int, int, hipStream_t)
 W4A16_WIDE(ActBf16, true);
@@ -557,6 +642,7 @@ W4A16_WIDE(ActF16, false);
 #undef W4A16_WIDE
 #define W4A16_WIDE_SWIGLU(PACKED)                                                          \
   template bool wide_serves<PACKED>(int, int, int);                                       \
+  template bool wide_slices_serve<PACKED>(const uint16_t*, int, int, int);                \
   template int launch_wide_swiglu<PACKED>(const uint8_t*, const uint16_t*, const uint8_t*, \
                                           const uint16_t*, const uint16_t*, uint16_t*, int, int, \
                                           int, hipStream_t)

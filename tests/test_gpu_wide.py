@@ -1,5 +1,5 @@
 """The 64 x 64 wave-tile GEMM (w4a16_gemm_wide.hip): shapes its dispatch rule
-takes on a 256-CU part, at the edges of its tiles. N not a multiple of 8 (one
+takes on a 256-CU part, its k-slice form among them, at the edges of its tiles. N not a multiple of 8 (one
 output per lane in the stores), of 32 or of 256, M one row past a tile, one
 group (K = 128), odd numbers of groups, K of several 8-group units with a
 short last one, file-layout scale rows that are not 4 B aligned. Outputs must
@@ -15,7 +15,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(51201, 128, 33), (25617, 384, 65), (3584, 1024, 897), (6152, 640, 513),
-          (5000, 1152, 700), (2056, 2176, 1473)]
+          (5000, 1152, 700), (2056, 2176, 1473),
+          # k-slices: four units, a short last one, three units, ragged N and M
+          (1024, 3584, 777), (1001, 2176, 600), (2040, 4096, 489), (8100, 2688, 100)]
 
 
 def _inputs(dev, N, K, M, dtype, seed):
