@@ -268,6 +268,51 @@ template <class Act, bool PACKED>
 int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                    int K, int M, hipStream_t stream);
 
+// Up to 8 projections sharing the activations x, for one launch of a prefill
+// kernel. Its row tiles are numbered over all projections in order; end[j] is
+// the first number past projection j's (set by the launch for its tile size).
+struct PrefillGroup {
+  const uint8_t* w[CUDALM_W4A16_MAX_PROJ];
+  const uint16_t* s[CUDALM_W4A16_MAX_PROJ];
+  uint16_t* y[CUDALM_W4A16_MAX_PROJ];
+  int n[CUDALM_W4A16_MAX_PROJ];
+  int end[CUDALM_W4A16_MAX_PROJ];
+  const uint16_t* x;
+  int count;
+};
+
+struct PrefillProj {
+  const uint8_t* w;
+  const uint16_t* s;
+  uint16_t* y;
+  int n;
+};
+
+// The projection that owns row tile t (uniform), t made relative to it. Every
+// field is read at a constant offset and chosen with scalar selects.
+__device__ __forceinline__ PrefillProj prefill_proj(const PrefillGroup& P, int& t) {
+  PrefillProj v = {P.w[0], P.s[0], P.y[0], P.n[0]};
+  int begin = 0;
+#pragma unroll
+  for (int j = 1; j < CUDALM_W4A16_MAX_PROJ; ++j) {
+    const bool past = j < P.count && t >= P.end[j - 1];
+    v.w = past ? P.w[j] : v.w;
+    v.s = past ? P.s[j] : v.s;
+    v.y = past ? P.y[j] : v.y;
+    v.n = past ? P.n[j] : v.n;
+    begin = past ? P.end[j - 1] : begin;
+  }
+  t -= begin;
+  return v;
+}
+
+template <bool PACKED>
+int launch_prefill_group(const PrefillGroup& P, int K, int M, hipStream_t stream);
+template <bool PACKED>
+bool wide_group_serves(const PrefillGroup& P, int K, int M);
+template <bool PACKED>
+int launch_wide_group(const PrefillGroup& P, int K, int M, hipStream_t stream);
+
 // Its 32 x 32 MFMA kernels alone: 32 activation rows x 256 weight rows per
 // 8-wave workgroup (at K = 1024 the split kernel).
 template <class Act, bool PACKED>

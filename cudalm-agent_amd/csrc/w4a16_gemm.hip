@@ -583,9 +583,11 @@ int launch_gemm32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16
 constexpr int kSliceMaxUnits = 4;  // units per k-slice kept as partials (KS > 1)
 
 template <class Act, int RB, int CT, int WV, bool PACKED, bool SVEC, int KS = 1, bool IOFF = false>
-__global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
-    const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
-    const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int K, int M) {
+__device__ __forceinline__ void gemm_unit_tile(const uint8_t* __restrict__ W,
+                                               const uint16_t* __restrict__ S,
+                                               const uint16_t* __restrict__ X,
+                                               uint16_t* __restrict__ Y, int N, int K, int M,
+                                               int bx) {
   constexpr int NT = WV * 64;  // threads of one k-slice
   constexpr int TM = CT * 16;
   constexpr int PB = x_pitch(kUnit * kGroup);  // LDS row pitch in 16-byte blocks (padded)
@@ -611,8 +613,8 @@ __global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
 
   int rt[RB];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) rt[rb] = min((blockIdx.x * WV + wave) * RB + rb, ntiles - 1);
-  const bool any_ok = (blockIdx.x * WV + wave) * RB < ntiles;
+  for (int rb = 0; rb < RB; ++rb) rt[rb] = min((bx * WV + wave) * RB + rb, ntiles - 1);
+  const bool any_ok = (bx * WV + wave) * RB < ntiles;
 
   // lane addresses of each owned tile at group 0
   const uint8_t* wbase[RB];
@@ -801,7 +803,7 @@ __global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
   if (!any_ok) return;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
-    const int n = ((blockIdx.x * WV + wave) * RB + rb) * kTileRows + i;
+    const int n = ((bx * WV + wave) * RB + rb) * kTileRows + i;
     if (n >= N) continue;
     uint16_t* col = Y + static_cast<size_t>(m0 + 4 * a) * N + n;
 #pragma unroll
@@ -813,6 +815,23 @@ __global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
               out_value<Act, PACKED>(total[rb][ct][r], W, S, K, n,
                                          X + static_cast<size_t>(m0 + ct * 16 + 4 * a + r) * K)));
   }
+}
+
+template <class Act, int RB, int CT, int WV, bool PACKED, bool SVEC, int KS = 1, bool IOFF = false>
+__global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
+    const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
+    const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int K, int M) {
+  gemm_unit_tile<Act, RB, CT, WV, PACKED, SVEC, KS, IOFF>(W, S, X, Y, N, K, M, blockIdx.x);
+}
+
+// Projections sharing x: blockIdx.x numbers the row tiles of all of them in
+// turn (P.end).
+template <int WV, bool PACKED, bool SVEC, int KS, bool IOFF>
+__global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_group_kernel(PrefillGroup P, int K,
+                                                                             int M) {
+  int bx = blockIdx.x;
+  const PrefillProj v = prefill_proj(P, bx);
+  gemm_unit_tile<ActBf16, 1, 2, WV, PACKED, SVEC, KS, IOFF>(v.w, v.s, P.x, v.y, v.n, K, M, bx);
 }
 
 template <class Act, int RB, int CT, int WV, bool PACKED, int KS = 1, bool IOFF = false>
@@ -913,6 +932,56 @@ int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint1
     return launch_gemm_unit<Act, 1, 2, 4, PACKED, 2, true>(W, S, X, Y, N, K, M, stream);
   return launch_gemm_unit<Act, 1, 2, 4, PACKED, 1, true>(W, S, X, Y, N, K, M, stream);
 }
+
+namespace {
+
+template <int WV, bool PACKED, int KS, bool IOFF>
+int launch_unit_group(PrefillGroup P, int K, int M, hipStream_t stream) {
+  const int U = (K / kGroup + kUnit - 1) / kUnit;
+  const size_t xbytes = static_cast<size_t>(32) * x_pitch(kUnit * kGroup) * 16;
+  if constexpr (KS > 1)
+    if (U > KS * kSliceMaxUnits || static_cast<size_t>(U) * WV * 2 * 64 * 16 > KS * xbytes)
+      return launch_unit_group<WV, PACKED, 1, IOFF>(P, K, M, stream);
+  const int gy = (M + 31) / 32;
+  if (gy > 65535) return CUDALM_W4A16_ERANGE;
+  bool svec = !PACKED && (K / kGroup) % 8 == 0;
+  int tiles = 0;
+  for (int j = 0; j < P.count; ++j) {
+    tiles += (P.n[j] + WV * kTileRows - 1) / (WV * kTileRows);
+    P.end[j] = tiles;
+    svec = svec && aligned(P.s[j], 16);
+  }
+  const size_t lds = KS * (xbytes + static_cast<size_t>(kUnit) * 32 * sizeof(float));
+  auto kern = svec ? w4a16_gemm_unit_group_kernel<WV, PACKED, !PACKED, KS, IOFF>
+                   : w4a16_gemm_unit_group_kernel<WV, PACKED, false, KS, IOFF>;
+  if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
+  hipLaunchKernelGGL(kern, dim3(tiles, gy), dim3(WV * KS * 64), lds, stream, P, K, M);
+  return launch_status();
+}
+
+}  // namespace
+
+// Projections sharing x, M >= 33, in one launch: the wide kernel or the unit
+// GEMM's tiles by the rules of launch_prefill on the tiles of all of them.
+// One call per projection took a launch of 5 us or more for each, the two of
+// 16 rows too. us, those calls first: qkv/z/b/a (6144, 2048, 16, 16 x 1024)
+// prepacked M = 33 18.1 / 6.6, 128 19.3 / 9.8, 512 28.0 / 19.2, 1024 41.4 / 29.1;
+// q/k/v (4096, 512, 512) M = 128 14.0 / 8.2, 777 23.8 / 18.4; gate/up (3584
+// twice) M = 64 9.4 / 7.2, 512 15.8 / 13.0, file layout 18.1 / 14.1; K = 4096
+// qkv/z/b/a M = 1024 128 / 101. No shape from M = 33 to 1024 and K = 512 to
+// 4096 measured slower.
+template <bool PACKED>
+int launch_prefill_group(const PrefillGroup& P, int K, int M, hipStream_t stream) {
+  if (wide_group_serves<PACKED>(P, K, M)) return launch_wide_group<PACKED>(P, K, M, stream);
+  long long wgs = 0;
+  for (int j = 0; j < P.count; ++j) wgs += (P.n[j] + 127) / 128;
+  wgs *= (M + 31) / 32;
+  if (5 * wgs >= 3LL * cu_count()) return launch_unit_group<8, PACKED, 1, false>(P, K, M, stream);
+  if (K > kUnit * kGroup) return launch_unit_group<4, PACKED, 2, true>(P, K, M, stream);
+  return launch_unit_group<4, PACKED, 1, true>(P, K, M, stream);
+}
+template int launch_prefill_group<true>(const PrefillGroup&, int, int, hipStream_t);
+template int launch_prefill_group<false>(const PrefillGroup&, int, int, hipStream_t);
 
 int prefill32_regs() { return regs_of(w4a16_gemm32_split_kernel<ActBf16, 8, true, false>); }
 int prefill_unit_regs() { return regs_of(w4a16_gemm_unit_kernel<ActBf16, 1, 2, 8, true, false>); }

@@ -86,10 +86,23 @@ struct WideArgs {
   int tiles_m, tiles_n;
 };
 
+struct WideGroupArgs {
+  PrefillGroup g;
+  int K, M;
+  int tiles_m, tiles_n;
+};
+
+// The operands of column tile bn, made relative to its projection.
+__device__ __forceinline__ const WideArgs& wide_view(const WideArgs& a, int&) { return a; }
+__device__ __forceinline__ WideArgs wide_view(const WideGroupArgs& a, int& bn) {
+  const PrefillProj v = prefill_proj(a.g, bn);
+  return WideArgs{{v.w, v.w}, {v.s, v.s}, a.g.x, v.y, v.n, a.K, a.M, a.tiles_m, a.tiles_n};
+}
+
 // SVEC: 4-byte aligned scale pairs (prepacked, or G even and S 4 B aligned)
 template <class Act, int MT, int NT, int WV, int OCC, bool PACKED, bool SVEC, bool MULTI, bool GLU,
-          int KS = 1>
-__global__ __launch_bounds__(WV * KS * 64, OCC) void w4a16_gemm_wide_kernel(WideArgs p) {
+          int KS = 1, class Args = WideArgs>
+__global__ __launch_bounds__(WV * KS * 64, OCC) void w4a16_gemm_wide_kernel(Args args) {
   static_assert(!GLU || NT == 2, "a wave holds a gate and an up tile");
   static_assert(KS == 1 || (!GLU && !MULTI), "a k-slice is one unit");
   constexpr int BM = 32 * MT;
@@ -102,7 +115,7 @@ __global__ __launch_bounds__(WV * KS * 64, OCC) void w4a16_gemm_wide_kernel(Wide
   u32x4_t* const xs = lds + slice * (wide_lds_bytes<MT>() / 16);
   float* const ob = reinterpret_cast<float*>(xs + 4 * XB);
 
-  const int K = p.K, N = p.N;
+  const int K = args.K;
   const int G = K >> 7;
   // this slice's groups: [gb, ge), all of them or one 8-group unit
   const int gb = slice * kUnit, ge = KS == 1 ? G : min(G, gb + kUnit);
@@ -115,18 +128,20 @@ __global__ __launch_bounds__(WV * KS * 64, OCC) void w4a16_gemm_wide_kernel(Wide
   // run of tiles, in bands of 8 tile rows walked column by column
   int bm, bn;
   {
-    const int total = p.tiles_m * p.tiles_n;
+    const int total = args.tiles_m * args.tiles_n;
     const int per = (total + 7) >> 3;
     const int L = blockIdx.x;
     const int idx = (L & 7) * per + (L >> 3);
     if ((L >> 3) >= per || idx >= total) return;
-    const int band = 8 * p.tiles_n;
+    const int band = 8 * args.tiles_n;
     const int bi = idx / band;
     const int rem = idx - bi * band;
-    const int rows = min(8, p.tiles_m - bi * 8);
+    const int rows = min(8, args.tiles_m - bi * 8);
     bn = rem / rows;
     bm = bi * 8 + rem - bn * rows;
   }
+  const WideArgs p = wide_view(args, bn);
+  const int N = p.N;
   const int m0 = bm * BM;
   const int mrows = min(BM, p.M - m0);
   const int nbase = (bn * WV + wave) * BNW;
@@ -549,6 +564,55 @@ bool wide_serves(int N, int K, int M) {
   const long long need = PACKED ? 25 : K <= kUnit * kGroup ? 20 : 12;  // 32nds of a tile per CU
   return t >= 0 && 32 * t >= need * cu_count();
 }
+
+// Projections sharing x: the same line on the tiles of all of them (their
+// single calls reach it later, if at all).
+template <bool PACKED>
+bool wide_group_serves(const PrefillGroup& P, int K, int M) {
+  long long t = 0;
+  for (int j = 0; j < P.count; ++j) {
+    const long long tj = wide_tiles(P.n[j], K, M, 64, 128);
+    if (tj < 0) return false;
+    t += static_cast<long long>((M + 63) / 64) * ((P.n[j] + 255) / 256);
+  }
+  const long long need = PACKED ? 25 : K <= kUnit * kGroup ? 20 : 12;
+  return t < (1LL << 28) && 32 * t >= need * cu_count();
+}
+
+template <int NT, bool PACKED, bool SVEC, bool MULTI>
+int launch_wide_group_t(WideGroupArgs a, hipStream_t stream) {
+  constexpr int BN = 4 * 32 * NT;
+  a.tiles_m = (a.M + 63) / 64;
+  a.tiles_n = 0;
+  for (int j = 0; j < a.g.count; ++j) {
+    a.tiles_n += (a.g.n[j] + BN - 1) / BN;
+    a.g.end[j] = a.tiles_n;
+  }
+  auto kern = w4a16_gemm_wide_kernel<ActBf16, 2, NT, 4, 2, PACKED, SVEC, MULTI, false, 1, WideGroupArgs>;
+  const size_t lds = wide_lds_bytes<2>();
+  if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
+  const int grid = 8 * ((a.tiles_m * a.tiles_n + 7) / 8);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, stream, a);
+  return launch_status();
+}
+
+template <bool PACKED>
+int launch_wide_group(const PrefillGroup& P, int K, int M, hipStream_t stream) {
+  const WideGroupArgs a = {P, K, M, 0, 0};
+  if constexpr (!PACKED) {
+    bool svec = (K / kGroup) % 2 == 0;
+    for (int j = 0; j < P.count; ++j) svec = svec && aligned(P.s[j], 4);
+    if (!svec)
+      return K <= kUnit * kGroup ? launch_wide_group_t<2, PACKED, false, false>(a, stream)
+                                 : launch_wide_group_t<1, PACKED, false, true>(a, stream);
+  }
+  return K <= kUnit * kGroup ? launch_wide_group_t<2, PACKED, true, false>(a, stream)
+                             : launch_wide_group_t<1, PACKED, true, true>(a, stream);
+}
+template bool wide_group_serves<true>(const PrefillGroup&, int, int);
+template bool wide_group_serves<false>(const PrefillGroup&, int, int);
+template int launch_wide_group<true>(const PrefillGroup&, int, int, hipStream_t);
+template int launch_wide_group<false>(const PrefillGroup&, int, int, hipStream_t);
 
 template <class Act, bool PACKED>
 int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,

@@ -2161,6 +2161,20 @@ int cudalm_w4a16_gemv_bf16_multi(const cudalm_w4a16_proj* projs, int count, cons
   if (prepacked && !vec_ok) return CUDALM_W4A16_EALIGN;
   long long tiles = 0;
   for (int j = 0; j < count; ++j) tiles += (projs[j].N + kTileRows - 1) / kTileRows;
+  if (vec_ok && count > 1 && M > 32 && tiles <= (1LL << 30) && M <= 65535 * 32) {
+    // a prefill chunk: one launch over the tiles of all projections
+    PrefillGroup g = {};
+    for (int j = 0; j < count; ++j) {
+      g.w[j] = static_cast<const uint8_t*>(projs[j].weight);
+      g.s[j] = projs[j].scale;
+      g.y[j] = projs[j].y;
+      g.n[j] = projs[j].N;
+    }
+    g.x = x;
+    g.count = count;
+    return prepacked ? launch_prefill_group<true>(g, K, M, stream)
+                     : launch_prefill_group<false>(g, K, M, stream);
+  }
   if (!vec_ok || tiles > (1LL << 30) ||
       (!stream_fits(K, M, prepacked) && !piece_direct(static_cast<int>(tiles), K, M))) {
     // not one fused launch: one call per projection (same bits)

@@ -99,7 +99,8 @@ int cudalm_w4a16_gemv_bf16_prepacked(const void* packed, const uint16_t* x,
  * q/k/v, in_proj_qkv/z/b/a and gate/up groups of a decoder layer,
  * src/runtime/qwen35_deltanet.cpp:166-181,236-243 and
  * src/runtime/qwen35_full_attention.cpp:211-240), computed by one launch
- * when M <= 32 and x fits on chip, else one launch per projection. Each
+ * when M > 32, or when M <= 32 and x fits on chip, else (and where a base is
+ * misaligned) by one launch per projection. Each
  * y_j is bit-identical to the single-projection call. No counterpart in the
  * reference (it issues one launch per projection). */
 #define CUDALM_W4A16_MAX_PROJ 8
@@ -222,9 +223,8 @@ int cudalm_w4a16_gemv_f16_prepacked(const void* packed, const uint16_t* x,
  * sequence gate -> up -> qwen35_silu_mul_bf16
  * (src/runtime/qwen35_deltanet.cpp:236-247) run on this library, with no
  * intermediate buffers. Any M (chunks of up to 32 rows, or the prefill GEMM
- * for larger M); all
- * bases 16 B aligned (y: 2 B), else EALIGN. No counterpart in the
- * reference. */
+ * for larger M); all bases 16 B aligned (y: 2 B), else EALIGN. No
+ * counterpart in the reference. */
 int cudalm_w4a16_swiglu_bf16(const void* gate_weight, const uint16_t* gate_scale,
                              const void* up_weight, const uint16_t* up_scale,
                              const uint16_t* x, uint16_t* y, int N, int K, int M,

@@ -117,3 +117,31 @@ def test_f16_prefill_equals_decode_kernels(w4, dev, N, K, M):
     y = torch.empty(M, N, dtype=torch.float16, device=dev)
     w4.gemv_f16(w, s, x, N, K, M, y=y)
     _same(y, ref, "file")
+
+
+@pytest.mark.parametrize("Ns,K,M", [((6144, 2048, 16, 16), 1024, 33), ((4096, 512, 512), 1024, 300),
+                                    ((3584, 3584), 1024, 577), ((1001, 37, 130), 640, 65),
+                                    ((512,) * 8, 2176, 70), ((1000, 16, 2049), 4096, 129),
+                                    ((1, 5000, 129, 3000), 128, 700), ((3000, 17), 9216, 40),
+                                    ((2056, 16, 2000), 2176, 1473)])
+def test_prefill_group_equals_single_calls(w4, dev, Ns, K, M):
+    # one launch over all projections' tiles: the unit GEMM's forms (two
+    # k-slices, more units than they keep) and the wide kernel's
+    ws, ss = [], []
+    for j, N in enumerate(Ns):
+        w, s, _ = _inputs(dev, N, K, 1, torch.bfloat16, 0x6E0 + j + K)
+        ws.append(w)
+        ss.append(s)
+    x = _inputs(dev, 1, K, M, torch.bfloat16, 0x6F0 + M)[2]
+    x[M // 2, 7] = float("inf")
+    packed = [w4.repack(w, s, N, K) for w, s, N in zip(ws, ss, Ns)]
+    refs = [w4.gemv_prepacked(p, x, N, K, M, y=torch.empty(M, N, dtype=torch.bfloat16, device=dev))
+            for p, N in zip(packed, Ns)]
+    buf = torch.empty(ss[0].numel() + 1, dtype=torch.float16, device=dev)
+    s2 = buf[1:].view_as(ss[0])  # one projection's scales off 4 bytes
+    s2.copy_(ss[0])
+    for label, got in (("prepacked", w4.gemv_multi(packed, None, x, Ns, K, M, prepacked=True)),
+                       ("file", w4.gemv_multi(ws, ss, x, Ns, K, M)),
+                       ("scales", w4.gemv_multi(ws, [s2] + ss[1:], x, Ns, K, M))):
+        for y, ref in zip(got, refs):
+            _same(y, ref, (label, ref.shape))
