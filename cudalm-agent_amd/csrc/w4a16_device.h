@@ -313,7 +313,15 @@ bool wide_group_serves(const PrefillGroup& P, int K, int M);
 template <bool PACKED>
 int launch_wide_group(const PrefillGroup& P, int K, int M, hipStream_t stream);
 
-// Its 32 x 32 MFMA kernels alone: 32 activation rows x 256 weight rows per
+// SwiGLU front half of M > 32 rows on GEMM tiles, and where those beat the
+// chunks of 32 rows.
+bool swiglu_gemm_serves(int N, int K, int M);
+template <bool PACKED>
+int launch_gemm_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
+                       const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,
+                       hipStream_t stream);
+
+// The 32 x 32 MFMA kernels of launch_prefill alone: 32 activation rows x 256 weight rows per
 // 8-wave workgroup (at K = 1024 the split kernel).
 template <class Act, bool PACKED>
 int launch_prefill32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
@@ -340,7 +348,7 @@ int launch_wide_slices(const uint8_t* W, const uint16_t* S, const uint16_t* X, u
                        int K, int M, hipStream_t stream);
 
 // The same kernel over gate and up, storing silu(gate) * up.
-bool wide_swiglu_serves(int N, int K, int M);
+bool wide_swiglu_fits(int N, int K, int M);
 template <bool PACKED>
 int launch_wide_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
                        const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,

@@ -582,12 +582,18 @@ int launch_gemm32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16
 
 constexpr int kSliceMaxUnits = 4;  // units per k-slice kept as partials (KS > 1)
 
-template <class Act, int RB, int CT, int WV, bool PACKED, bool SVEC, int KS = 1, bool IOFF = false>
+// GLU: RB = 2, the wave's tiles are the same rows of gate (W, S) and up (W2,
+// S2), and y = silu(gate) * up is stored.
+template <class Act, int RB, int CT, int WV, bool PACKED, bool SVEC, int KS = 1, bool IOFF = false,
+          bool GLU = false>
 __device__ __forceinline__ void gemm_unit_tile(const uint8_t* __restrict__ W,
                                                const uint16_t* __restrict__ S,
                                                const uint16_t* __restrict__ X,
                                                uint16_t* __restrict__ Y, int N, int K, int M,
-                                               int bx) {
+                                               int bx, const uint8_t* __restrict__ W2 = nullptr,
+                                               const uint16_t* __restrict__ S2 = nullptr) {
+  static_assert(!GLU || RB == 2, "a gate and an up tile");
+  constexpr int TR = GLU ? 1 : RB;  // output tiles per wave
   constexpr int NT = WV * 64;  // threads of one k-slice
   constexpr int TM = CT * 16;
   constexpr int PB = x_pitch(kUnit * kGroup);  // LDS row pitch in 16-byte blocks (padded)
@@ -613,8 +619,8 @@ __device__ __forceinline__ void gemm_unit_tile(const uint8_t* __restrict__ W,
 
   int rt[RB];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) rt[rb] = min((bx * WV + wave) * RB + rb, ntiles - 1);
-  const bool any_ok = (bx * WV + wave) * RB < ntiles;
+  for (int rb = 0; rb < RB; ++rb) rt[rb] = min((bx * WV + wave) * TR + (GLU ? 0 : rb), ntiles - 1);
+  const bool any_ok = (bx * WV + wave) * TR < ntiles;
 
   // lane addresses of each owned tile at group 0
   const uint8_t* wbase[RB];
@@ -622,13 +628,13 @@ __device__ __forceinline__ void gemm_unit_tile(const uint8_t* __restrict__ W,
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     if constexpr (PACKED) {
-      const uint8_t* tile = W + static_cast<size_t>(rt[rb]) * packed_tile_bytes(G);
+      const uint8_t* tile = (GLU && rb == 1 ? W2 : W) + static_cast<size_t>(rt[rb]) * packed_tile_bytes(G);
       wbase[rb] = tile + lane * 16;
       sbase[rb] = tile + static_cast<size_t>(G) * 1024 + i * packed_scale_pitch(G);
     } else {
       const int row = min(rt[rb] * kTileRows + i, N - 1);
-      wbase[rb] = W + static_cast<size_t>(row) * (K >> 1) + a * 16;
-      sbase[rb] = reinterpret_cast<const uint8_t*>(S + static_cast<size_t>(row) * G);
+      wbase[rb] = (GLU && rb == 1 ? W2 : W) + static_cast<size_t>(row) * (K >> 1) + a * 16;
+      sbase[rb] = reinterpret_cast<const uint8_t*>((GLU && rb == 1 ? S2 : S) + static_cast<size_t>(row) * G);
     }
   }
   constexpr int kStep = PACKED ? 1024 : 64;  // bytes between groups of one lane
@@ -801,6 +807,22 @@ __device__ __forceinline__ void gemm_unit_tile(const uint8_t* __restrict__ W,
       }
   }
   if (!any_ok) return;
+  if constexpr (GLU) {
+    const int n = rt[0] * kTileRows + i;
+    if (n >= N) return;
+    uint16_t* col = Y + static_cast<size_t>(m0 + 4 * a) * N + n;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (ct * 16 + 4 * a + r < mrows) {
+          const uint16_t* xrow = X + static_cast<size_t>(m0 + ct * 16 + 4 * a + r) * K;
+          const uint32_t gt = Act::round(out_value<Act, PACKED>(total[0][ct][r], W, S, K, n, xrow));
+          const uint32_t up = Act::round(out_value<Act, PACKED>(total[1][ct][r], W2, S2, K, n, xrow));
+          col[static_cast<size_t>(ct * 16 + r) * N] = static_cast<uint16_t>(silu_mul_bits(gt, up));
+        }
+    return;
+  }
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int n = ((bx * WV + wave) * RB + rb) * kTileRows + i;
@@ -822,6 +844,15 @@ __global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_kernel(
     const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
     const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, int N, int K, int M) {
   gemm_unit_tile<Act, RB, CT, WV, PACKED, SVEC, KS, IOFF>(W, S, X, Y, N, K, M, blockIdx.x);
+}
+
+template <int WV, bool PACKED, bool SVEC, int KS, bool IOFF>
+__global__ __launch_bounds__(WV * KS * 64) void w4a16_gemm_unit_swiglu_kernel(
+    const uint8_t* __restrict__ Wg, const uint8_t* __restrict__ Wu, const uint16_t* __restrict__ X,
+    int N, int K, int M, const uint16_t* __restrict__ Sg, const uint16_t* __restrict__ Su,
+    uint16_t* __restrict__ Y) {
+  gemm_unit_tile<ActBf16, 2, 2, WV, PACKED, SVEC, KS, IOFF, true>(Wg, Sg, X, Y, N, K, M, blockIdx.x,
+                                                                 Wu, Su);
 }
 
 // Projections sharing x: blockIdx.x numbers the row tiles of all of them in
@@ -959,6 +990,27 @@ int launch_unit_group(PrefillGroup P, int K, int M, hipStream_t stream) {
   return launch_status();
 }
 
+template <int WV, bool PACKED, int KS, bool IOFF>
+int launch_unit_swiglu_t(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
+                         const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,
+                         hipStream_t stream) {
+  const int U = (K / kGroup + kUnit - 1) / kUnit;
+  const size_t xbytes = static_cast<size_t>(32) * x_pitch(kUnit * kGroup) * 16;
+  if constexpr (KS > 1)
+    if (U > KS * kSliceMaxUnits || static_cast<size_t>(U) * WV * 4 * 64 * 16 > KS * xbytes)
+      return launch_unit_swiglu_t<WV, PACKED, 1, IOFF>(Wg, Sg, Wu, Su, X, Y, N, K, M, stream);
+  const int gx = (N + WV * kTileRows - 1) / (WV * kTileRows), gy = (M + 31) / 32;
+  if (gy > 65535) return CUDALM_W4A16_ERANGE;
+  const bool svec = !PACKED && (K / kGroup) % 8 == 0 && aligned(Sg, 16) && aligned(Su, 16);
+  const size_t lds = KS * (xbytes + static_cast<size_t>(kUnit) * 32 * sizeof(float));
+  auto kern = svec ? w4a16_gemm_unit_swiglu_kernel<WV, PACKED, !PACKED, KS, IOFF>
+                   : w4a16_gemm_unit_swiglu_kernel<WV, PACKED, false, KS, IOFF>;
+  if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
+  hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(WV * KS * 64), lds, stream, Wg, Wu, X, N, K, M, Sg, Su,
+                     Y);
+  return launch_status();
+}
+
 }  // namespace
 
 // Projections sharing x, M >= 33, in one launch: the wide kernel or the unit
@@ -982,6 +1034,48 @@ int launch_prefill_group(const PrefillGroup& P, int K, int M, hipStream_t stream
 }
 template int launch_prefill_group<true>(const PrefillGroup&, int, int, hipStream_t);
 template int launch_prefill_group<false>(const PrefillGroup&, int, int, hipStream_t);
+
+// SwiGLU of M > 32 rows: GEMM tiles against the chunked kernels, whose 16 x 32
+// tiles take a workgroup each. Theirs / the unit GEMM's tiles, us, by their
+// workgroups on 256 CUs, prepacked: K = 1024: 128 (512, M = 128) 6.3 / 6.6, 256
+// (1024, M = 128) 6.7 / 6.8, 448 (3584, M = 64) 11.8 / 7.0, 896 (M = 128) 21.9 /
+// 7.3; K = 512: 376 (3001, M = 64) 7.1 / 5.9, file layout 7.1 / 6.6, M = 40 6.3 /
+// 6.7; K = 2048: 192 (1024, M = 96) 8.5 / 10.2, 256 (M = 128) 15.4 / 10.3; K =
+// 3584: 128 (1024, M = 64) 13.2 / 15.6, 192 (M = 96) 24.7 / 15.7.
+bool swiglu_gemm_serves(int N, int K, int M) {
+  if (M <= 32) return false;
+  const long long tiles = static_cast<long long>((N + 15) / 16) * ((M + 31) / 32);
+  const long long cus = cu_count();
+  if (K <= kUnit * kGroup) return 2 * tiles >= 3 * cus;
+  return K <= 2 * kUnit * kGroup ? tiles >= cus : 4 * tiles >= 3 * cus;
+}
+
+// The unit GEMM's 128 x 32 tiles (a gate and an up tile per wave) while they
+// make one round, then the wide kernel (3584 x 1024: M = 256, 224 tiles, 9.4 us
+// against 13.1; M = 384, 336 tiles, 17.0 / 13.4; M = 1000 22.3 for the wide one,
+// 143.5 in chunks; K = 2048: M = 256 14.4 / 23, M = 512 27.7 / 23.0). Below 3/5
+// of a round 64 x 32 tiles, with two k-slices past K = 1024, as in
+// launch_prefill.
+template <bool PACKED>
+int launch_gemm_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
+                       const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,
+                       hipStream_t stream) {
+  const long long wgs = static_cast<long long>((N + 127) / 128) * ((M + 31) / 32);
+  const long long cus = cu_count();
+  if (wgs > cus && wide_swiglu_fits(N, K, M))
+    return launch_wide_swiglu<PACKED>(Wg, Sg, Wu, Su, X, Y, N, K, M, stream);
+  if (5 * wgs >= 3 * cus)
+    return launch_unit_swiglu_t<8, PACKED, 1, false>(Wg, Sg, Wu, Su, X, Y, N, K, M, stream);
+  if (K > kUnit * kGroup)
+    return launch_unit_swiglu_t<4, PACKED, 2, true>(Wg, Sg, Wu, Su, X, Y, N, K, M, stream);
+  return launch_unit_swiglu_t<4, PACKED, 1, true>(Wg, Sg, Wu, Su, X, Y, N, K, M, stream);
+}
+template int launch_gemm_swiglu<true>(const uint8_t*, const uint16_t*, const uint8_t*,
+                                      const uint16_t*, const uint16_t*, uint16_t*, int, int, int,
+                                      hipStream_t);
+template int launch_gemm_swiglu<false>(const uint8_t*, const uint16_t*, const uint8_t*,
+                                       const uint16_t*, const uint16_t*, uint16_t*, int, int, int,
+                                       hipStream_t);
 
 int prefill32_regs() { return regs_of(w4a16_gemm32_split_kernel<ActBf16, 8, true, false>); }
 int prefill_unit_regs() { return regs_of(w4a16_gemm_unit_kernel<ActBf16, 1, 2, 8, true, false>); }

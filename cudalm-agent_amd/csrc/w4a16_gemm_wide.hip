@@ -498,7 +498,9 @@ __global__ __launch_bounds__(WV * KS * 64, OCC) void w4a16_gemm_wide_kernel(Args
         if constexpr (GLU) {
           const float own = nt == 0 ? f[0] : f[1];
           if (own == own) continue;
-          const float e = w4a16_ref_dot<PACKED>(p.w[nt], p.s[nt], K, n, xrow);
+          // (no dynamic index into the argument copy: that would live in scratch)
+          const float e = w4a16_ref_dot<PACKED>(nt == 0 ? p.w[0] : p.w[1], nt == 0 ? p.s[0] : p.s[1],
+                                                K, n, xrow);
           // gate first (q ascending): up's turn recomputes gate if it was NaN too
           float g = nt == 0 ? e : f[0];
           const float u = nt == 0 ? f[1] : e;
@@ -659,23 +661,7 @@ int launch_wide_slices(const uint8_t* W, const uint16_t* S, const uint16_t* X, u
   return launch_wide_t<Act, 1, 1, 4, 1, PACKED, true, false, false, 4>(p, stream);
 }
 
-// SwiGLU: against the chunked kernels' 16 x 32 tiles (a workgroup each). The
-// wide kernel takes one round (12-13 us at K = 1024, 23 at 2048, 36 at 3584)
-// up to a tile of 64 x 128 per CU, theirs grow by the workgroup. us, theirs
-// against this kernel's:
-//   K = 1024: 448 tiles (3584, M = 64) 11.8 / 13.0, 512 (512, M = 512)
-//     11.5 / 12.7, 672 (3584, M = 96) 17.0 / 13.1, 2048 (16384, M = 64)
-//     19.2 / 14
-//   K = 512: 564 (3001, M = 96) 10.5 / 11.1, 1316 (M = 200) 16.8 / 11.2
-//   K = 2048: 512 (1024, M = 256) 22.7 / 23.0, 1024 (M = 512) 42.2 / 23.0
-//   K = 3584: 448 (3584, M = 64) 44 / 35.5, 672 (M = 96) 60 / 35.5
-// M <= 32 (one chunk) always stays with them.
-bool wide_swiglu_serves(int N, int K, int M) {
-  if (M <= 32 || wide_tiles(N, K, M, 64, 128) < 0) return false;
-  const long long tiles = static_cast<long long>((N + 15) / 16) * ((M + 31) / 32);
-  const long long cus = cu_count();
-  return K <= 2 * kUnit * kGroup ? 4 * tiles >= 9 * cus : 2 * tiles >= 3 * cus;
-}
+bool wide_swiglu_fits(int N, int K, int M) { return wide_tiles(N, K, M, 64, 128) >= 0; }
 
 template <bool PACKED>
 int launch_wide_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,

@@ -1886,8 +1886,8 @@ int launch_swiglu(const ProjTable& P, const uint16_t* X, int K, int M, hipStream
   const bool svec = !PACKED && G % 8 == 0 && aligned(P.s[0], 16) && aligned(P.s[1], 16);
   // (what no chunk of the fused kernel serves stays refused below)
   const int mu = swiglu_rows_per_chunk(K, M);
-  if (mu >= 1 && (M + mu - 1) / mu <= 65535 && wide_swiglu_serves(P.n[0], K, M))
-    return launch_wide_swiglu<PACKED>(P.w[0], P.s[0], P.w[1], P.s[1], X, P.y[0], P.n[0], K, M, stream);
+  if (mu >= 1 && (M + mu - 1) / mu <= 65535 && swiglu_gemm_serves(P.n[0], K, M))
+    return launch_gemm_swiglu<PACKED>(P.w[0], P.s[0], P.w[1], P.s[1], X, P.y[0], P.n[0], K, M, stream);
   const SplitPlan plan = swiglu_piece_plan(P.tile_end[0], K, M);
   if (plan.hg != 0) {
     int mc = M > 16 ? 32 : M;

@@ -6,7 +6,7 @@ short last one, file-layout scale rows that are not 4 B aligned. Outputs must
 equal, bit for bit, those of calls of at most 32 rows, which the decode
 kernels serve (every row of a batched call equals the single-row call on it),
 for bf16 and fp16 activations, both weight layouts, non-finite activations,
-and for the SwiGLU form of the kernel; the bf16 outputs also the forced tile
+and for the SwiGLU forms of it and of the unit GEMM; the bf16 outputs also the forced tile
 kernel's."""
 import numpy as np
 import pytest
@@ -82,9 +82,14 @@ def test_wide_equals_decode_kernels(w4, dev, N, K, M, f16):
     _same(y, ref, "output base")
 
 
-@pytest.mark.parametrize("N,K,M", [(3584, 1024, 100), (3584, 1024, 833), (8200, 384, 70),
-                                   (16385, 128, 40), (2048, 2176, 300), (3000, 3584, 65)])
-def test_wide_swiglu_equals_chunks(w4, dev, N, K, M):
+@pytest.mark.parametrize("N,K,M", [(3584, 1024, 833), (8200, 384, 190), (16385, 128, 129),
+                                   (2048, 2176, 600), (3000, 3584, 700),  # wide kernel
+                                   # unit GEMM: 128- and 64-row tiles, two k-slices, more
+                                   # units than the slices keep, ragged N
+                                   (3584, 1024, 100), (8200, 384, 70), (3001, 512, 40),
+                                   (6001, 640, 33), (1030, 3584, 97), (1024, 2048, 129),
+                                   (1029, 9216, 100)])
+def test_gemm_swiglu_equals_chunks(w4, dev, N, K, M):
     gw, gs, x = _inputs(dev, N, K, M, torch.bfloat16, 0x51F + N + M)
     uw, us, _ = _inputs(dev, N, K, 1, torch.bfloat16, 0x520 + K)
     gp, up = w4.repack(gw, gs, N, K), w4.repack(uw, us, N, K)
