@@ -295,9 +295,18 @@ int launch_stream(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int 
                   hipStream_t stream) {
   const int mc = stream_rows_per_chunk(K, M);
   if (mc < 1) return CUDALM_W4A16_EVARIANT;
-  if (prefer_gemm(N, K, M, mc, PACKED)) return launch_bf16_gemm<PACKED>(W, X, Y, N, K, M, stream);
   if (mc > 16) return launch_stream_ct<2, PACKED>(W, X, Y, N, K, M, mc, stream);
   return launch_stream_ct<1, PACKED>(W, X, Y, N, K, M, mc, stream);
+}
+
+// What an ordinary call runs: the GEMM where it is faster, else the stream kernel.
+template <bool PACKED = false>
+int launch_auto(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int K, int M,
+                hipStream_t stream) {
+  const int mc = stream_rows_per_chunk(K, M);
+  if (mc >= 1 && prefer_gemm(N, K, M, mc, PACKED))
+    return launch_bf16_gemm<PACKED>(W, X, Y, N, K, M, stream);
+  return launch_stream<PACKED>(W, X, Y, N, K, M, stream);
 }
 
 // One thread per 16-byte chunk of the tile-major layout.
@@ -351,7 +360,7 @@ int cudalm_bf16_gemv_variant(const uint16_t* weight, const uint16_t* x, uint16_t
   const bool vec = stream_ok(weight, x, K, M);
   switch (variant) {
     case CUDALM_BF16_VARIANT_AUTO:
-      return vec ? launch_stream(weight, x, y, N, K, M, stream)
+      return vec ? launch_auto(weight, x, y, N, K, M, stream)
                  : launch_scalar(weight, x, y, N, K, M, stream);
     case CUDALM_BF16_VARIANT_STREAM:
       if (!vec) return CUDALM_W4A16_EVARIANT;
@@ -391,7 +400,7 @@ int cudalm_bf16_gemv_prepacked(const void* packed, const uint16_t* x, uint16_t* 
   if (N % kTile != 0 || K % kUnitK != 0) return CUDALM_W4A16_EINVAL;
   if (!aligned(packed, 16) || !aligned(x, 16) || !aligned(y, 2)) return CUDALM_W4A16_EALIGN;
   if (stream_rows_per_chunk(K, M) < 1) return CUDALM_W4A16_EVARIANT;
-  return launch_stream<true>(static_cast<const uint16_t*>(packed), x, y, N, K, M, stream);
+  return launch_auto<true>(static_cast<const uint16_t*>(packed), x, y, N, K, M, stream);
 }
 
 int cudalm_bf16_gemv_kernel_regs(int variant) {

@@ -45,6 +45,8 @@ def test_gemm_equals_stream_kernel(w4, dev, N, K, M, spread):
         y = torch.empty_like(ref)
         w4.bf16_gemv_any(w, x, N, K, M, y=y)
         _same(y, ref, ("file", bad))
+        w4.bf16_gemv_any(w, x, N, K, M, y=y, variant="stream")  # the chunks, forced
+        _same(y, ref, ("stream", bad))
         if N % 16 == 0 and K % 256 == 0:
             y = torch.empty_like(ref)
             w4.bf16_gemv_prepacked(w4.bf16_repack(w, N, K), x, N, K, M, y=y)
