@@ -1994,27 +1994,36 @@ bool piece_direct(int ntiles, int K, int M) {
   return p.hg != 0 && p.dx;
 }
 
+// 17 <= M <= 32 at long K, where x leaves room for one workgroup per CU or does
+// not fit the LDS at all: the prefill kernels, which stage it by units, unless a
+// split kernel serves the call (a tile per CU at most) or the tiles are so
+// many that the streamed weights bound both. us, stream kernel (two 16-row
+// passes where x does not fit) / prefill kernels, prepacked: 6144 x 2432 M = 17
+// 12.9 / 9.6, 16384 x 2432 M = 32 14.5 / 10.7, 60000 x 2432 M = 32 21.8 / 26.2,
+// 2048 x 2432 M = 32 (no room for the split) 13.9 / 9.7; not fitting: 6144 x
+// 3584 M = 32 27.1 / 11.0, 16384 x 4096 M = 24 24.6 / 13.4, 60000 x 4096 M = 32
+// 62.4 / 41.3. The piece split keeps 4096 x 4096 M = 17 8.7 / 11.5, M = 32
+// 11.3 / 11.4.
+bool prefer_prefill(int ntiles, int K, int M, bool packed) {
+  if (M <= 16 || M > 32) return false;
+  if (!stream_fits(K, M, packed)) return !piece_direct(ntiles, K, M);
+  if (K <= 2 * kUnit * kGroup) return false;
+  if (ntiles <= cu_count()) return !split_fits(K, M, packed) && !piece_direct(ntiles, K, M);
+  return ntiles <= 4 * cu_count();
+}
+
 template <bool PACKED>
 int dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
              int M, int variant, hipStream_t stream) {
   if (variant == CUDALM_W4A16_VARIANT_AUTO) {
-    if (stream_fits(K, M, PACKED) || piece_direct((N + kTileRows - 1) / kTileRows, K, M)) {
+    const int ntiles = (N + kTileRows - 1) / kTileRows;
+    if (M > 32 || prefer_prefill(ntiles, K, M, PACKED)) {
+      variant = CUDALM_W4A16_VARIANT_PREFILL;
+    } else if (stream_fits(K, M, PACKED) || piece_direct(ntiles, K, M)) {
       const ProjTable P = single_table(W, S, Y, N);
       return launch_stream<PACKED>(P, X, K, M, stream);
-    } else if (M <= 32 && M > 16) {
-      // x does not fit in LDS at once: 16-row column passes
-      for (int m0 = 0; m0 < M; m0 += 16) {
-        const int mc = M - m0 < 16 ? M - m0 : 16;
-        if (int rc = dispatch<PACKED>(W, S, X + static_cast<size_t>(m0) * K,
-                                      Y + static_cast<size_t>(m0) * N, N, K, mc,
-                                      CUDALM_W4A16_VARIANT_AUTO, stream))
-          return rc;
-      }
-      return CUDALM_W4A16_OK;
-    } else if (M <= 16) {
-      variant = CUDALM_W4A16_VARIANT_TILE16;
     } else {
-      variant = CUDALM_W4A16_VARIANT_PREFILL;
+      variant = CUDALM_W4A16_VARIANT_TILE16;
     }
   }
   switch (variant) {
@@ -2053,7 +2062,11 @@ int f16_dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_
   int mc = M < 32 ? M : 32;
   while (mc > 0 && !stream_fits(K, mc, PACKED)) --mc;
   if (mc < 1) return CUDALM_W4A16_ERANGE;
-  if (M > 32 && M <= 65535 * 32) return launch_prefill<ActF16, PACKED>(W, S, X, Y, N, K, M, stream);
+  // (mc < M <= 32: two launches of the stream kernels, 4096 x 3584 M = 32 15.5 us
+  // against 10.9)
+  if (M <= 65535 * 32 && (M > 32 || (M > 16 && mc < M) ||
+                          prefer_prefill((N + kTileRows - 1) / kTileRows, K, M, PACKED)))
+    return launch_prefill<ActF16, PACKED>(W, S, X, Y, N, K, M, stream);
   for (int m0 = 0; m0 < M; m0 += mc) {
     const int rows = M - m0 < mc ? M - m0 : mc;
     const ProjTable P = single_table(W, S, Y + static_cast<size_t>(m0) * N, N);
@@ -2161,8 +2174,10 @@ int cudalm_w4a16_gemv_bf16_multi(const cudalm_w4a16_proj* projs, int count, cons
   if (prepacked && !vec_ok) return CUDALM_W4A16_EALIGN;
   long long tiles = 0;
   for (int j = 0; j < count; ++j) tiles += (projs[j].N + kTileRows - 1) / kTileRows;
-  if (vec_ok && count > 1 && M > 32 && tiles <= (1LL << 30) && M <= 65535 * 32) {
-    // a prefill chunk: one launch over the tiles of all projections
+  const bool prefill = vec_ok && tiles <= (1LL << 30) && M <= 65535 * 32 &&
+                       (M > 32 || prefer_prefill(static_cast<int>(tiles), K, M, prepacked));
+  if (prefill && count > 1) {
+    // the prefill kernels: one launch over the tiles of all projections
     PrefillGroup g = {};
     for (int j = 0; j < count; ++j) {
       g.w[j] = static_cast<const uint8_t*>(projs[j].weight);
@@ -2175,7 +2190,7 @@ int cudalm_w4a16_gemv_bf16_multi(const cudalm_w4a16_proj* projs, int count, cons
     return prepacked ? launch_prefill_group<true>(g, K, M, stream)
                      : launch_prefill_group<false>(g, K, M, stream);
   }
-  if (!vec_ok || tiles > (1LL << 30) ||
+  if (!vec_ok || tiles > (1LL << 30) || prefill ||
       (!stream_fits(K, M, prepacked) && !piece_direct(static_cast<int>(tiles), K, M))) {
     // not one fused launch: one call per projection (same bits)
     for (int j = 0; j < count; ++j) {

@@ -99,8 +99,8 @@ int cudalm_w4a16_gemv_bf16_prepacked(const void* packed, const uint16_t* x,
  * q/k/v, in_proj_qkv/z/b/a and gate/up groups of a decoder layer,
  * src/runtime/qwen35_deltanet.cpp:166-181,236-243 and
  * src/runtime/qwen35_full_attention.cpp:211-240), computed by one launch
- * when M > 32, or when M <= 32 and x fits on chip, else (and where a base is
- * misaligned) by one launch per projection. Each
+ * for any M; where a base is misaligned, or M <= 16 and x does not fit on
+ * chip, by one launch per projection. Each
  * y_j is bit-identical to the single-projection call. No counterpart in the
  * reference (it issues one launch per projection). */
 #define CUDALM_W4A16_MAX_PROJ 8

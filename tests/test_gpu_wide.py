@@ -150,3 +150,30 @@ def test_prefill_group_equals_single_calls(w4, dev, Ns, K, M):
                        ("scales", w4.gemv_multi(ws, [s2] + ss[1:], x, Ns, K, M))):
         for y, ref in zip(got, refs):
             _same(y, ref, (label, ref.shape))
+
+
+@pytest.mark.parametrize("N,K,M", [(6144, 2432, 17), (4113, 2304, 32), (2048, 2432, 32),
+                                   (5001, 3584, 25), (60001, 4096, 31), (1000, 9216, 32),
+                                   (4096, 3584, 32)])
+def test_long_k_batches_equal_sixteen_row_calls(w4, dev, N, K, M):
+    # 17 to 32 rows whose x fills the LDS or does not fit it: the prefill
+    # kernels, against calls of at most 16 rows
+    for dtype, packed_call, file_call in ((torch.bfloat16, w4.gemv_prepacked, w4.gemv),
+                                          (torch.float16, w4.gemv_f16_prepacked, w4.gemv_f16)):
+        w, s, x = _inputs(dev, N, K, M, dtype, 0x10F + N + K + M)
+        p = w4.repack(w, s, N, K)
+        x[M - 1, 5] = float("nan")
+        ref = torch.empty(M, N, dtype=dtype, device=dev)
+        for m0 in range(0, M, 16):
+            xc = x[m0:m0 + 16].contiguous()
+            packed_call(p, xc, N, K, xc.shape[0], y=ref[m0:m0 + 16])
+        y = torch.empty_like(ref)
+        packed_call(p, x, N, K, M, y=y)
+        _same(y, ref, "prepacked")
+        y = torch.empty_like(ref)
+        file_call(w, s, x, N, K, M, y=y)
+        _same(y, ref, "file")
+        if dtype == torch.bfloat16:
+            for ns in (1, 2):
+                for y in w4.gemv_multi([p] * ns, None, x, [N] * ns, K, M, prepacked=True):
+                    _same(y, ref, ("group", ns))
