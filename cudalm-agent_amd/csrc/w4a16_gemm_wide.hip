@@ -550,35 +550,81 @@ long long wide_tiles(int N, int K, int M, int bm, int bn) {
   return t < (1LL << 30) ? t : -1;
 }
 
-}  // namespace
-
-// Where the 64 x 256 tiles beat the smaller-tiled prefill kernels (both in
-// us, theirs first; t = tiles on 256 CUs). Prepacked: from 25/32 of a tile
-// per CU: K = 1024 t = 182 12.2 / 12.4, 192 12.2 / 12.5, 208 15.0 / 12.8, 312
-// 19.1 / 18.7, 768 42.3 / 29.8; K = 3584 t = 112 25.2 / 25.6, 208 44.6 / 35.0.
-// File layout, whose loads the smaller tiles repeat more often: from 5/8 at
-// K <= 1024 (t = 128 9.6 / 9.7, 182 14.1 / 13.2, 768 46.8 / 32.3) and from 3/8
-// beyond (K = 2048 t = 96 17.0 / 15.5, 64 11.5 / 13.8; K = 3584 t = 104 33.6 /
-// 25.7).
-template <bool PACKED>
-bool wide_serves(int N, int K, int M) {
-  const long long t = wide_tiles(N, K, M, 64, 256);
-  const long long need = PACKED ? 25 : K <= kUnit * kGroup ? 20 : 12;  // 32nds of a tile per CU
-  return t >= 0 && 32 * t >= need * cu_count();
+// Where the wide kernel beats the smaller-tiled prefill kernels. Two lines, in
+// us below, theirs first.
+//
+// A fill line on 64 x 256 tiles (t of them on 256 CUs). Prepacked: 25/32 of a
+// tile per CU: K = 1024 t = 182 12.2 / 12.4, 192 12.2 / 12.5, 208 15.0 / 12.8,
+// 768 42.3 / 29.8; K = 3584 t = 112 25.2 / 25.6, 208 44.6 / 35.0. File layout,
+// whose loads the smaller tiles repeat more often: 5/8 at K <= 1024 (t = 128
+// 9.6 / 9.7, 182 14.1 / 13.2, 768 46.8 / 32.3) and 3/8 beyond (K = 2048 t = 96
+// 17.0 / 15.5, 64 11.5 / 13.8; K = 3584 t = 104 33.6 / 25.7).
+//
+// Both sides then step by rounds of one workgroup per CU: w of this kernel's
+// tiles (64 x 256, 64 x 128 past K = 1024) and s of the 128 x 32 ones, and a
+// ragged M or N, which this kernel pads further, costs it rounds they do not
+// take. Medians over 2,000 random shapes by round, K = 1024 prepacked: s = 2 9.8,
+// 3 15, 4 21, 5 24, 6 30, 7 34; w = 1 13.5, 2 23, 3 32. File layout s = 2 11, 3
+// 16, 4 20, 5 24, 6 28, 7 34; w = 1 14.5, 2 25, 3 35. So at K <= 1024 s > 2 w
+// (K = 1024 file layout N = 20342, M = 80 10.0 / 13.9; N = 41863, M = 65 19.2 /
+// 23.4); at most K = 256 prepacked, 512 file layout, where s = 4 equals w = 2,
+// s >= 2 w, and K <= 256 file layout keeps the fill line alone (s = 2 8.3, w = 1
+// 7.3). Past K = 1024, K = 2048 prepacked: s = 2 17.5, 3 24.8, 4 34, 5 40, 6 47, 7
+// 54; w = 1 17, 2 26, 3 39, 4 50: 2 s >= 3 w (N = 50045, M = 72 39.9 / 48.4),
+// which also holds for file-layout scales that are loaded a unit at a time
+// (K a multiple of 1024: N = 19595, M = 65 19.1 / 24.4). Those loaded one by
+// one slow the smaller tiles (K = 3584: s = 2 35, 3 51, 4 67, 5 81; w = 1 26.5,
+// 2 39.5, 3 61, 4 78): 3 s >= 4 w.
+//
+// A narrow matrix (N <= 64) leaves half of a 128 x 32 tile's waves or more
+// without rows, and counts half a tile (K = 1024 prepacked N = 19, M = 16391
+// 9.4 / 18.1; file layout K = 2048 N = 17, M = 7735 8.0 / 16.6); in a group, where
+// the other projections' tiles share the CU with it, three quarters, and a whole
+// one at K <= 512 (K = 1024 file layout (18, 23, 33), M = 11605: one call per
+// projection 20.1 / 29.1).
+bool wide_rounds_pay(bool packed, int K, long long wide, long long small8) {
+  const long long cus = cu_count();
+  const long long w = (wide + cus - 1) / cus;
+  const long long s = (small8 + 8 * cus - 1) / (8 * cus);  // small8: eighths of a tile
+  if (K > kUnit * kGroup)
+    return packed || (K / kGroup) % kUnit == 0 ? 2 * s >= 3 * w : 3 * s >= 4 * w;
+  if (!packed && K <= 2 * kGroup) return true;
+  if (K <= (packed ? 2 : 4) * kGroup) return s >= 3 && s >= 2 * w;
+  return s > 2 * w;
 }
 
-// Projections sharing x: the same line on the tiles of all of them (their
-// single calls reach it later, if at all).
+// 32nds of a 64 x 256 tile per CU that make the fill line
+template <bool PACKED>
+int wide_fill(int K) {
+  return PACKED ? 25 : K <= kUnit * kGroup ? 20 : 12;
+}
+
+int wide_tile_cols(int K) { return K <= kUnit * kGroup ? 256 : 128; }
+
+}  // namespace
+
+template <bool PACKED>
+bool wide_serves(int N, int K, int M) {
+  const long long t = wide_tiles(N, K, M, 64, 256), wide = wide_tiles(N, K, M, 64, wide_tile_cols(K));
+  if (t < 0 || wide < 0 || 32 * t < wide_fill<PACKED>(K) * cu_count()) return false;
+  const long long cols8 = N <= 64 ? 4 : 8LL * ((N + 127) / 128);
+  return wide_rounds_pay(PACKED, K, wide, (M + 31) / 32 * cols8);
+}
+
+// Projections sharing x: the same lines on the tiles of all of them (their
+// single calls reach them later, if at all).
 template <bool PACKED>
 bool wide_group_serves(const PrefillGroup& P, int K, int M) {
-  long long t = 0;
+  long long t = 0, wide = 0, cols8 = 0;
   for (int j = 0; j < P.count; ++j) {
-    const long long tj = wide_tiles(P.n[j], K, M, 64, 128);
-    if (tj < 0) return false;
-    t += static_cast<long long>((M + 63) / 64) * ((P.n[j] + 255) / 256);
+    const int N = P.n[j], bn = wide_tile_cols(K);
+    if (wide_tiles(N, K, M, 64, 128) < 0) return false;
+    t += static_cast<long long>((M + 63) / 64) * ((N + 255) / 256);
+    wide += static_cast<long long>((M + 63) / 64) * ((N + bn - 1) / bn);
+    cols8 += N <= 64 && K > 4 * kGroup ? 6 : 8LL * ((N + 127) / 128);
   }
-  const long long need = PACKED ? 25 : K <= kUnit * kGroup ? 20 : 12;
-  return t < (1LL << 28) && 32 * t >= need * cu_count();
+  if (t >= (1LL << 28) || 32 * t < wide_fill<PACKED>(K) * cu_count()) return false;
+  return wide_rounds_pay(PACKED, K, wide, (M + 31) / 32 * cols8);
 }
 
 template <int NT, bool PACKED, bool SVEC, bool MULTI>

@@ -1,0 +1,61 @@
+"""Which kernel the dispatch rules pick on a 256-CU part, at shapes where both
+sides were timed: the wide GEMM's rules at ragged and narrow shapes, where a
+rule on its own tiles alone had taken calls that the smaller tiles serve
+faster, and beside them shapes that it keeps."""
+import pytest
+import torch
+
+from launched_kernels import launched_kernels
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _part(dev):
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the shapes stand at the rules' lines of a 256-CU part")
+
+
+def _weights(dev, N, K):
+    return (torch.zeros(N, K // 2, dtype=torch.uint8, device=dev),
+            torch.ones(N, K // 128, dtype=torch.float16, device=dev))
+
+
+def _x(dev, M, K):
+    return torch.zeros(M, K, dtype=torch.bfloat16, device=dev)
+
+
+@pytest.mark.parametrize("packed,N,K,M,kernel", [
+    # M one row into a second 64-row tile, or a third 32-row one
+    (False, 20342, 1024, 80, "gemm32_split"), (False, 41863, 1024, 65, "gemm_unit"),
+    (False, 22110, 1024, 160, "gemm_unit"), (False, 19595, 2048, 65, "gemm_unit"),
+    (True, 50045, 2048, 72, "gemm_unit"), (True, 40335, 3584, 72, "gemm_unit"),
+    # N of a few rows, very many activation rows
+    (True, 19, 1024, 16391, "gemm32_split"), (False, 17, 2048, 7735, "gemm_unit"),
+    # what the wide kernel keeps, ragged sizes among them
+    (False, 6144, 1024, 2048, "gemm_wide"), (True, 4096, 1024, 1024, "gemm_wide"),
+    (True, 248320, 1024, 256, "gemm_wide"), (False, 22420, 512, 129, "gemm_wide"),
+    (False, 3584, 3584, 777, "gemm_wide"), (True, 6152, 640, 513, "gemm_wide")])
+def test_prefill_kernel(w4, dev, packed, N, K, M, kernel):
+    w, s = _weights(dev, N, K)
+    x, y = _x(dev, M, K), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    if packed:
+        p = w4.repack(w, s, N, K)
+        names = launched_kernels(lambda: w4.gemv_prepacked(p, x, N, K, M, y=y))
+    else:
+        names = launched_kernels(lambda: w4.gemv(w, s, x, N, K, M, y=y))
+    assert len(names) == 1 and kernel in names[0], names
+
+
+@pytest.mark.parametrize("packed,Ns,K,M,kernel", [
+    (False, (18, 23, 33), 1024, 11605, "gemm_unit"), (True, (28, 47), 1024, 8091, "gemm_unit"),
+    (True, (6144, 2048, 16, 16), 1024, 1024, "gemm_wide"),
+    (False, (3584, 3584), 1024, 512, "gemm_wide")])
+def test_prefill_group_kernel(w4, dev, packed, Ns, K, M, kernel):
+    pairs = [_weights(dev, N, K) for N in Ns]
+    x = _x(dev, M, K)
+    ys = [torch.empty(M, N, dtype=torch.bfloat16, device=dev) for N in Ns]
+    ws = [w4.repack(w, s, N, K) if packed else w for (w, s), N in zip(pairs, Ns)]
+    ss = None if packed else [s for _, s in pairs]
+    names = launched_kernels(lambda: w4.gemv_multi(ws, ss, x, Ns, K, M, ys=ys, prepacked=packed))
+    assert len(names) == 1 and kernel in names[0], names
