@@ -687,14 +687,22 @@ int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t
 // Below one round of 64 x 32 tiles (M = 512: 12.9 against 14.7 us) and at
 // short K the unit GEMM is faster (K = 2048, two slices, M = 777 9.9 against
 // 10.6 us; prepacked 4096 x 2304, M = 256 11.1 against 11.5, file layout 14.7
-// against 12.6). What
+// against 12.6). Three units (prepacked 2560 < K <= 3072) leave one slice idle,
+// and where the 128 x 32 tiles are what the unit GEMM would run, it is as fast or
+// faster when the column tiles are even in number: they are numbered first, so a
+// workgroup's XCD (its number % 8) then keeps to half, a quarter or an eighth of
+// the weights. Slices / unit GEMM, median and range over 2,200 random shapes:
+// odd 0.92 (0.80 - 1.07), even 1.02 (0.84 - 1.12), from 25/32 of a round 0.95;
+// multiples of four 1.06 (0.82 - 1.18; 3050 x 3072, M = 276 15.2 / 13.1 us). What
 // bounds the slices is VALU: at 32 rows a decoded dword feeds one MFMA.
 template <bool PACKED>
 bool wide_slices_serve(const uint16_t* S, int N, int K, int M) {
   if (K <= (PACKED ? 20 * kGroup : 2 * kUnit * kGroup) || K > 4 * kUnit * kGroup) return false;
   if (!PACKED && (K / kGroup) % 8 == 0 && aligned(S, 16)) return false;
-  const long long rows = (M + 31) / 32, cus = cu_count();
-  return rows * ((N + 63) / 64) > cus && rows * ((N + 127) / 128) <= cus;
+  const long long rows = (M + 31) / 32, cols = (N + 127) / 128, cus = cu_count();
+  if (rows * ((N + 63) / 64) <= cus || rows * cols > cus) return false;
+  if (!PACKED || K > 3 * kUnit * kGroup || 5 * rows * cols < 3 * cus) return true;
+  return cols % 2 != 0 || (cols % 4 != 0 && 32 * rows * cols >= 25 * cus);
 }
 
 template <class Act, bool PACKED>

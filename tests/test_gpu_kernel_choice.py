@@ -35,7 +35,11 @@ def _x(dev, M, K):
     # what the wide kernel keeps, ragged sizes among them
     (False, 6144, 1024, 2048, "gemm_wide"), (True, 4096, 1024, 1024, "gemm_wide"),
     (True, 248320, 1024, 256, "gemm_wide"), (False, 22420, 512, 129, "gemm_wide"),
-    (False, 3584, 3584, 777, "gemm_wide"), (True, 6152, 640, 513, "gemm_wide")])
+    (False, 3584, 3584, 777, "gemm_wide"), (True, 6152, 640, 513, "gemm_wide"),
+    # its k-slices over three units: column tiles even in number, odd, and few
+    # 128 x 32 tiles
+    (True, 3050, 3072, 276, "gemm_unit"), (True, 1130, 3072, 768, "gemm_wide"),
+    (True, 2216, 2816, 227, "gemm_wide"), (True, 1024, 3584, 777, "gemm_wide")])
 def test_prefill_kernel(w4, dev, packed, N, K, M, kernel):
     w, s = _weights(dev, N, K)
     x, y = _x(dev, M, K), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
