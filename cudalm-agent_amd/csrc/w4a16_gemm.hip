@@ -1041,12 +1041,24 @@ template int launch_prefill_group<false>(const PrefillGroup&, int, int, hipStrea
 // (1024, M = 128) 6.7 / 6.8, 448 (3584, M = 64) 11.8 / 7.0, 896 (M = 128) 21.9 /
 // 7.3; K = 512: 376 (3001, M = 64) 7.1 / 5.9, file layout 7.1 / 6.6, M = 40 6.3 /
 // 6.7; K = 2048: 192 (1024, M = 96) 8.5 / 10.2, 256 (M = 128) 15.4 / 10.3; K =
-// 3584: 128 (1024, M = 64) 13.2 / 15.6, 192 (M = 96) 24.7 / 15.7.
-bool swiglu_gemm_serves(int N, int K, int M) {
+// 3584: 128 (1024, M = 64) 13.2 / 15.6, 192 (M = 96) 24.7 / 15.7. (At K <= 1024 the
+// line lies where hardly a shape loses, not where the gains begin: M = 64 gains
+// from fewer tiles than M = 40, and file layout 3784 x 640, M = 35, 474 tiles, 6.7 /
+// 7.5, still does not.)
+//
+// Past K = 1024 a chunk's workgroups have a CU each, and while all of them fit
+// one round the chunks are the faster: 1024 x 1152, M = 109 file layout, 256
+// workgroups, 7.8 / 11.4, 306 x 2304, M = 359 15.2 / 20.3, 434 x 2816, M = 221
+// prepacked 13.9 / 15.6. (How many rows a chunk has, and so how many workgroups
+// there are, follows from the LDS: 25 to 32 up to K = 2304, 17 at K = 4096.) Of 1,500
+// random shapes past K = 1024 three lose by 4 to 14 %, where the last chunk has
+// two to four rows.
+bool swiglu_gemm_serves(int N, int K, int M, int chunks) {
   if (M <= 32) return false;
-  const long long tiles = static_cast<long long>((N + 15) / 16) * ((M + 31) / 32);
+  const long long cols = (N + 15) / 16, tiles = cols * ((M + 31) / 32);
   const long long cus = cu_count();
   if (K <= kUnit * kGroup) return 2 * tiles >= 3 * cus;
+  if (cols * chunks <= cus) return false;
   return K <= 2 * kUnit * kGroup ? tiles >= cus : 4 * tiles >= 3 * cus;
 }
 

@@ -1884,27 +1884,29 @@ template <bool PACKED>
 int launch_swiglu(const ProjTable& P, const uint16_t* X, int K, int M, hipStream_t stream) {
   const int G = K / kGroup;
   const bool svec = !PACKED && G % 8 == 0 && aligned(P.s[0], 16) && aligned(P.s[1], 16);
+  // the piece kernel's chunk rows (a plan for M > 16 needs 32-row chunks, CT = 2)
+  const SplitPlan plan = swiglu_piece_plan(P.tile_end[0], K, M);
+  int mp = plan.hg == 0 ? 0 : M > 16 ? 32 : M;
+  while (mp > 0 && split_piece_lds_bytes(K, mp, plan, 2) > kLdsMax) --mp;
+  if (M > 16 && mp <= 16) mp = 0;
   // (what no chunk of the fused kernel serves stays refused below)
   const int mu = swiglu_rows_per_chunk(K, M);
-  if (mu >= 1 && (M + mu - 1) / mu <= 65535 && swiglu_gemm_serves(P.n[0], K, M))
+  const int rows = mp > 0 ? mp : mu;
+  if (mu >= 1 && (M + mu - 1) / mu <= 65535 &&
+      swiglu_gemm_serves(P.n[0], K, M, (M + rows - 1) / rows))
     return launch_gemm_swiglu<PACKED>(P.w[0], P.s[0], P.w[1], P.s[1], X, P.y[0], P.n[0], K, M, stream);
-  const SplitPlan plan = swiglu_piece_plan(P.tile_end[0], K, M);
-  if (plan.hg != 0) {
-    int mc = M > 16 ? 32 : M;
-    while (mc > 0 && split_piece_lds_bytes(K, mc, plan, 2) > kLdsMax) --mc;
-    // a plan for M > 16 needs 32-row chunks (CT = 2)
-    if (mc > 0 && (M <= 16 || mc > 16)) {
+  if (mp > 0) {
+    const int mc = mp;
 #define W4A16_SWP(NR, CT, HG, WV, DX)                                                      \
   (svec ? launch_swiglu_piece_t<PACKED, NR, true, CT, HG, WV, DX>(P, X, K, M, mc, stream) \
         : launch_swiglu_piece_t<PACKED, NR, false, CT, HG, WV, DX>(P, X, K, M, mc, stream))
-      if (mc > 16)
-        return plan.wv == 16 ? W4A16_SWP(4, 2, 2, 16, false) : W4A16_SWP(4, 2, 2, 8, false);
-      if (M == 1) return plan.dx ? W4A16_SWP(1, 1, 2, 8, true) : W4A16_SWP(1, 1, 4, 4, false);
-      return plan.dx ? W4A16_SWP(4, 1, 2, 8, true) : W4A16_SWP(4, 1, 4, 4, false);
+    if (mc > 16)
+      return plan.wv == 16 ? W4A16_SWP(4, 2, 2, 16, false) : W4A16_SWP(4, 2, 2, 8, false);
+    if (M == 1) return plan.dx ? W4A16_SWP(1, 1, 2, 8, true) : W4A16_SWP(1, 1, 4, 4, false);
+    return plan.dx ? W4A16_SWP(4, 1, 2, 8, true) : W4A16_SWP(4, 1, 4, 4, false);
 #undef W4A16_SWP
-    }
   }
-  const int mc = swiglu_rows_per_chunk(K, M);
+  const int mc = mu;
   if (mc < 1) return CUDALM_W4A16_ERANGE;
 #define W4A16_SWIGLU(NR, CT)                                                       \
   (svec ? launch_swiglu_t<PACKED, NR, true, CT>(P, X, K, M, mc, stream)           \

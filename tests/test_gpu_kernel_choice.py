@@ -63,3 +63,19 @@ def test_prefill_group_kernel(w4, dev, packed, Ns, K, M, kernel):
     ss = None if packed else [s for _, s in pairs]
     names = launched_kernels(lambda: w4.gemv_multi(ws, ss, x, Ns, K, M, ys=ys, prepacked=packed))
     assert len(names) == 1 and kernel in names[0], names
+
+
+@pytest.mark.parametrize("packed,N,K,M,kernel", [
+    # the chunks' workgroups fit one round
+    (False, 1024, 1152, 109, "split_piece_pair"), (False, 306, 2304, 359, "w4a16_swiglu"),
+    (True, 434, 2816, 221, "w4a16_swiglu"),
+    # they take two
+    (True, 1112, 2560, 102, "gemm_unit_swiglu"), (False, 1024, 1152, 130, "gemm_unit_swiglu"),
+    (True, 3584, 1024, 64, "gemm_unit_swiglu"), (True, 3584, 1024, 1000, "gemm_wide")])
+def test_swiglu_kernel(w4, dev, packed, N, K, M, kernel):
+    (gw, gs), (uw, us) = _weights(dev, N, K), _weights(dev, N, K)
+    if packed:
+        gw, uw, gs, us = w4.repack(gw, gs, N, K), w4.repack(uw, us, N, K), None, None
+    x, y = _x(dev, M, K), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    names = launched_kernels(lambda: w4.swiglu(gw, gs, uw, us, x, N, K, M, y=y, prepacked=packed))
+    assert len(names) == 1 and kernel in names[0], names
