@@ -282,12 +282,26 @@ int launch_stream_ct(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, i
 // 512 7.2 / 7.0, 1024 11.9 / 9.4; tile-major copy, K = 1024: 512 (16384, M =
 // 64) 9.9 / 11.3, 768 (M = 96) 18.1 / 14.9; K = 3072 (24-row chunks, one workgroup per
 // CU): 176 (1024, M = 256) 22.6 / 34.7, 384 (8192, M = 64) 39.4 / 26.3.
+//
+// Past K = 1024 the chunks' time steps by rounds of one workgroup per CU; a
+// short last chunk costs less than a round, and counts by its rows at M > 64 of
+// the tile-major copy (4160 x 2304, M = 101, 260 workgroups, 22.5 / 28.6; 864 x
+// 3840, M = 362, 266, 34.5 / 45.2). The GEMM takes 11 us per 1024 k while its tiles
+// fit one round, a round of chunks of the few rows that the LDS holds at long K
+// about half of that, so at M > 64 the chunks' second round still ties with it at
+// K = 4096, and is the faster one past that for the tile-major copy (3072 x 4352,
+// M = 111, 336, 44.2 / 51.0; 2016 x 5632, M = 108, 288, 46.3 / 64.7; 1280 x 7680, M =
+// 131, 280, 62.2 / 86.7) and past K = 8192 for the file layout, whose chunks load
+// slower (1152 x 8640, M = 158, 360, 79.0 / 96.4; below it 5 to 20 % either way, e.g.
+// 1511 x 7288, M = 180, 73.9 / 83.3, 425 x 6928, M = 423, 87.5 / 79.5).
 bool prefer_gemm(int N, int K, int M, int mc, bool packed) {
   if (M <= 32 || !bf16_gemm_fits(N, M)) return false;
-  const long long wgs = static_cast<long long>((N + 63) / 64) * ((M + mc - 1) / mc);
+  const long long cols = (N + 63) / 64, wgs = cols * ((M + mc - 1) / mc);
   const long long cus = cu_count();
-  if (K > 1024) return wgs > cus;
-  return wgs >= (M <= 64 && !packed ? 2 : 3) * cus;
+  if (K <= 1024) return wgs >= (M <= 64 && !packed ? 2 : 3) * cus;
+  if (M > 64 && K > (packed ? 4096 : 8192)) return wgs > 2 * cus;
+  if (M > 64 && packed && cols * M <= cus * mc) return false;
+  return wgs > cus;
 }
 
 template <bool PACKED = false>

@@ -1,7 +1,7 @@
 """Which kernel the dispatch rules pick on a 256-CU part, at shapes where both
-sides were timed: the wide GEMM's rules at ragged and narrow shapes, where a
-rule on its own tiles alone had taken calls that the smaller tiles serve
-faster, and beside them shapes that it keeps."""
+sides were timed: where a rule on the new kernel's own tiles alone (the wide
+GEMM and its k-slices, the SwiGLU GEMM, the bf16 GEMM) had taken calls that the
+kernel beside it serves faster, and beside them shapes that it keeps."""
 import pytest
 import torch
 
@@ -78,4 +78,24 @@ def test_swiglu_kernel(w4, dev, packed, N, K, M, kernel):
         gw, uw, gs, us = w4.repack(gw, gs, N, K), w4.repack(uw, us, N, K), None, None
     x, y = _x(dev, M, K), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
     names = launched_kernels(lambda: w4.swiglu(gw, gs, uw, us, x, N, K, M, y=y, prepacked=packed))
+    assert len(names) == 1 and kernel in names[0], names
+
+
+@pytest.mark.parametrize("packed,N,K,M,kernel", [
+    # a round of chunks and a few rows more, two rounds of long K
+    (True, 4160, 2304, 101, "gemv_stream"), (True, 864, 3840, 362, "gemv_stream"),
+    (True, 3072, 4352, 111, "gemv_stream"), (True, 2016, 5632, 108, "gemv_stream"),
+    (True, 1280, 7680, 131, "gemv_stream"), (False, 1152, 8640, 158, "gemv_stream"),
+    # enough of them, and 64-row tiles
+    (True, 2800, 2304, 192, "bf16_gemm"), (True, 8192, 5632, 108, "bf16_gemm"),
+    (False, 8192, 3072, 64, "bf16_gemm"), (True, 8704, 2304, 64, "bf16_gemm"),
+    (False, 248320, 1024, 64, "bf16_gemm")])
+def test_bf16_head_kernel(w4, dev, packed, N, K, M, kernel):
+    w = torch.zeros(N, K, dtype=torch.bfloat16, device=dev)
+    x, y = _x(dev, M, K), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    if packed:
+        p = w4.bf16_repack(w, N, K)
+        names = launched_kernels(lambda: w4.bf16_gemv_prepacked(p, x, N, K, M, y=y))
+    else:
+        names = launched_kernels(lambda: w4.bf16_gemv_any(w, x, N, K, M, y=y))
     assert len(names) == 1 and kernel in names[0], names
