@@ -254,6 +254,8 @@ int stream_wgs_per_cu() { return 4; }
 template <int CT, bool PACKED = false>
 int launch_stream_ct(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int K, int M,
                      int mc, hipStream_t stream) {
+  const int gy = (M + mc - 1) / mc;
+  if (gy > 65535) return CUDALM_W4A16_ERANGE;
   const size_t lds = stream_lds(K, mc);
   auto kern = bf16_gemv_stream_kernel<CT, PACKED>;
   if (!allow_lds(kern, lds)) return CUDALM_W4A16_ELAUNCH;
@@ -266,8 +268,6 @@ int launch_stream_ct(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, i
   const int rounds = (ntiles + cap_waves - 1) / cap_waves;
   const int waves = (ntiles + rounds - 1) / rounds;
   const int gx = (waves + kWaves - 1) / kWaves;
-  const int gy = (M + mc - 1) / mc;
-  if (gy > 65535) return CUDALM_W4A16_ERANGE;
   hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(kWaves * 64), lds, stream, W, X, Y, N, K, M, mc);
   return launch_status();
 }
@@ -313,12 +313,13 @@ int launch_stream(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int 
   return launch_stream_ct<1, PACKED>(W, X, Y, N, K, M, mc, stream);
 }
 
-// What an ordinary call runs: the GEMM where it is faster, else the stream kernel.
+// What an ordinary call runs: the GEMM where it is faster, else the stream
+// kernel, which refuses more chunks than its grid can number; so do both.
 template <bool PACKED = false>
 int launch_auto(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int K, int M,
                 hipStream_t stream) {
   const int mc = stream_rows_per_chunk(K, M);
-  if (mc >= 1 && prefer_gemm(N, K, M, mc, PACKED))
+  if (mc >= 1 && (M + mc - 1) / mc <= 65535 && prefer_gemm(N, K, M, mc, PACKED))
     return launch_bf16_gemm<PACKED>(W, X, Y, N, K, M, stream);
   return launch_stream<PACKED>(W, X, Y, N, K, M, stream);
 }

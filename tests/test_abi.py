@@ -107,6 +107,15 @@ def test_bf16_gemv_preconditions_rejected_before_device(w4):
     assert p(fake, fake, fake, 1 << 30, 16, 1) == w4.ERANGE
 
 
+def test_bf16_gemv_more_row_chunks_than_a_grid(w4):
+    # K = 40960 leaves one activation row per chunk: 65536 rows are refused,
+    # by both entry points and the forced stream variant
+    fake, N, K, M = 0x1000, 64, 40960, 65536
+    assert w4.bf16_gemv_ptr(fake, fake, fake, N, K, M) == w4.ERANGE
+    assert w4.bf16_gemv_ptr(fake, fake, fake, N, K, M, w4.BF16_VARIANT_STREAM) == w4.ERANGE
+    assert w4.lib().cudalm_bf16_gemv_prepacked(fake, fake, fake, N, K, M, None) == w4.ERANGE
+
+
 def test_bf16_repack_preconditions_rejected_before_device(w4):
     # include/cudalm_bf16_gemv.h: the packed path needs N % 16 == 0,
     # K % 256 == 0 and 16-byte aligned bases
