@@ -14,8 +14,8 @@
 // each stream the weights again (same box):
 //   M = 33 180 -> 102 / 174 -> 93, M = 64 188 -> 110 / 187 -> 100,
 //   M = 128 372 -> 126 / 367 -> 115, M = 256 744 -> 199 / 728 -> 193.
-// Three stages of loads in flight instead of two: 5 % slower (fewer waves
-// resident); 64-wide n per wave at M <= 64: 4x (spills); 256 x 128 tiles of 8
+// Three register sets of loads in flight instead of two (D = 3): 5 % slower (fewer
+// waves resident); 64-wide n per wave at M <= 64: 4x (spills); 256 x 128 tiles of 8
 // waves: level at M = 256, 174 us at M = 128.
 //
 // Same bits as the decode kernel: a 16 x 16 x 32 MFMA step over k-blocks
@@ -25,8 +25,9 @@
 //
 // Work decomposition. A workgroup of 4 waves owns 64 x 128 outputs (M <= 64:
 // 64 x 32 per wave) or 128 x 128 (64 x 64 per wave). Both operands go through
-// double-buffered LDS in 64-k stages, loaded to registers two stages ahead in
-// whole 128-byte lines (tile-major copy: whole 1 KB slabs). Tiles of one
+// double-buffered LDS in 64-k stages, in whole 128-byte lines (tile-major copy:
+// whole 1 KB slabs). Two register sets of loads are in flight (D = 2): a stage is
+// requested three stages before its turn and put into LDS one before it. Tiles of one
 // weight row block run on neighbouring workgroups of one XCD, so that its
 // second reader finds it in that XCD's L2.
 
@@ -36,16 +37,10 @@
 
 #include "bf16_gemm.h"
 #include "hip_common.h"
+#include "w4a16_device.h"
 
 namespace cudalm_hip {
 namespace {
-
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 
 constexpr int kBK = 64;           // k per stage
 constexpr int kBlocks = kBK / 8;  // 16-byte blocks per row and stage
@@ -155,7 +150,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void bf16_gemm_kernel(
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = mfma32(A[mt], B[nt], acc[mt][nt]);
+        for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = mfma32<ActBf16>(A[mt], B[nt], acc[mt][nt]);
     }
   };
 

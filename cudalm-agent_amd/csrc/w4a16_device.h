@@ -262,8 +262,8 @@ __device__ __forceinline__ uint32_t silu_mul_bits(uint32_t g_bits, uint32_t u_bi
   return mul_bits(silu_bits(g_bits), u_bits);
 }
 
-// GEMM of M >= 33 activation rows (w4a16_gemm.hip), the kernel chosen by
-// shape, for any N, M and K % 128 == 0.
+// GEMM of many activation rows (w4a16_gemm.hip; M >= 33, and 17 to 32 rows of
+// long K), the kernel chosen by shape, for any N, M and K % 128 == 0.
 template <class Act, bool PACKED>
 int launch_prefill(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N,
                    int K, int M, hipStream_t stream);
@@ -332,15 +332,20 @@ int launch_prefill32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uin
 int prefill32_regs();
 int prefill_unit_regs();
 
-// GEMM on 64 x 64 wave tiles (w4a16_gemm_wide.hip), for M and N large enough
-// to give every CU a workgroup of 64 x 256 outputs.
+// GEMM on 64 x 64 wave tiles (w4a16_gemm_wide.hip; 64 x 32 past K = 1024), and
+// whether it is the faster one: 64 x 256 tiles for 25/32 of the CUs (prepacked),
+// 20/32 (file layout, K <= 1024) or 12/32 (beyond), and few enough rounds of its
+// workgroups beside those of the smaller tiles.
 template <bool PACKED>
 bool wide_serves(int N, int K, int M);
 template <class Act, bool PACKED>
 int launch_wide(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y, int N, int K,
                 int M, hipStream_t stream);
 
-// Its form with k-slices of one unit each, for few tiles of 2048 < K <= 4096.
+// Its form with four k-slices of one unit each, for more than one round of 64 x
+// 32 tiles and at most one of 128 x 32: prepacked 2560 < K <= 4096 (up to 3072 by
+// the number of column tiles too), file layout 2048 < K <= 4096 where a unit's
+// scales cannot be loaded at once (K / 128 not a multiple of 8, or scales off 16 B).
 template <bool PACKED>
 bool wide_slices_serve(const uint16_t* S, int N, int K, int M);
 template <class Act, bool PACKED>

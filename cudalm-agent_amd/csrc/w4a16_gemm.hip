@@ -1,4 +1,9 @@
-// Prefill-chunk W4A16 GEMM on 32 x 32 MFMA tiles (MI355X, gfx950).
+// Prefill-chunk W4A16 GEMM (MI355X, gfx950): the kernels on 32 x 32 MFMA tiles
+// (one per call, and the K = 1024 one whose groups two wave sets share), the unit
+// GEMM on 16 x 16 tiles with its forms for a group of projections and for SwiGLU,
+// and launch_prefill and its like, which choose among them and the wide kernel
+// (w4a16_gemm_wide.hip). This header describes the 32 x 32 kernels; the unit GEMM
+// has its own further down.
 //
 // Contract (reference: tests/cuda/test_int4_gemv_bf16.cpp:54-69 applied row
 // by row; the reference itself runs prefill one token at a time,
@@ -928,8 +933,9 @@ int launch_prefill32(const uint8_t* W, const uint16_t* S, const uint16_t* X, uin
   return launch_gemm32<Act, 8, 1, 1, PACKED>(W, S, X, Y, N, K, M, stream);
 }
 
-// Prefill chunks (M >= 33). Shapes with enough 64 x 256 output tiles take
-// the wide kernel (wide_serves). The 32 x 32 MFMA GEMM (32 activation rows x
+// Prefill chunks (M >= 33, and 17 to 32 rows of long K). Shapes with enough 64 x
+// 256 output tiles that pad little take the wide kernel (wide_serves), few tiles of
+// long K its k-slices (wide_slices_serve). The 32 x 32 MFMA GEMM (32 activation rows x
 // 256 weight rows per 8-wave workgroup) serves K <= 1024
 // when its workgroups fill between 3/4 and all of the CUs in one round
 // (3584x1024 and 4096x1024 at M = 512: 10.3 -> 9.6-9.9 us, 10.7 -> 9.5-10.0 us);

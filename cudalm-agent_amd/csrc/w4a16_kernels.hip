@@ -2004,7 +2004,9 @@ bool piece_direct(int ntiles, int K, int M) {
 // 12.9 / 9.6, 16384 x 2432 M = 32 14.5 / 10.7, 60000 x 2432 M = 32 21.8 / 26.2,
 // 2048 x 2432 M = 32 (no room for the split) 13.9 / 9.7; not fitting: 6144 x
 // 3584 M = 32 27.1 / 11.0, 16384 x 4096 M = 24 24.6 / 13.4, 60000 x 4096 M = 32
-// 62.4 / 41.3. The piece split keeps 4096 x 4096 M = 17 8.7 / 11.5, M = 32
+// 64.0 / 31.5. Past K = 4096, 512 x 5120 M = 17 26.0 / 15.0, 2048 x 6144 M = 24 46.2 /
+// 16.8, 512 x 9216 M = 17 42.3 / 26.8, M = 32 68.3 / 27.0; of 2,000 random calls of N
+// <= 2048, K from 4096 to 10240, none is slower. The piece split keeps 4096 x 4096 M = 17 8.7 / 11.5, M = 32
 // 11.3 / 11.4.
 bool prefer_prefill(int ntiles, int K, int M, bool packed) {
   if (M <= 16 || M > 32) return false;
@@ -2064,8 +2066,8 @@ int f16_dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_
   int mc = M < 32 ? M : 32;
   while (mc > 0 && !stream_fits(K, mc, PACKED)) --mc;
   if (mc < 1) return CUDALM_W4A16_ERANGE;
-  // (mc < M <= 32: two launches of the stream kernels, 4096 x 3584 M = 32 15.5 us
-  // against 10.9)
+  // (mc < M <= 32: two or more launches of the stream kernels, 4096 x 3584 M = 32
+  // 15.5 us against 10.9, 512 x 9216 M = 17 31.8 / 27.6)
   if (M <= 65535 * 32 && (M > 32 || (M > 16 && mc < M) ||
                           prefer_prefill((N + kTileRows - 1) / kTileRows, K, M, PACKED)))
     return launch_prefill<ActF16, PACKED>(W, S, X, Y, N, K, M, stream);

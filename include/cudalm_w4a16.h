@@ -255,7 +255,8 @@ int cudalm_w4a16_dequant_f32(const uint8_t* weight, const uint16_t* scale,
 #define CUDALM_W4A16_VARIANT_STREAM 1   /* M <= 32, x resident in LDS */
 #define CUDALM_W4A16_VARIANT_TILE16 2   /* 16 columns per wave, K chunked */
 #define CUDALM_W4A16_VARIANT_TILE32 3   /* 32 columns per wave, K chunked */
-#define CUDALM_W4A16_VARIANT_PREFILL 4  /* prefill GEMM chosen by shape (M >= 33) */
+#define CUDALM_W4A16_VARIANT_PREFILL 4  /* prefill GEMM chosen by shape (AUTO: M >= 33,
+                                           and 17 to 32 rows of long K) */
 #define CUDALM_W4A16_VARIANT_BYTEWISE 5 /* misaligned-base fallback */
 #define CUDALM_W4A16_VARIANT_SPLIT 6    /* M <= 32, units of a tile on separate waves */
 #define CUDALM_W4A16_VARIANT_SWIGLU 7   /* kernel_regs only: the fused SwiGLU kernel */
