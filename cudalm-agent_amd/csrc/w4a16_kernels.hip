@@ -1889,10 +1889,10 @@ int launch_swiglu(const ProjTable& P, const uint16_t* X, int K, int M, hipStream
   int mp = plan.hg == 0 ? 0 : M > 16 ? 32 : M;
   while (mp > 0 && split_piece_lds_bytes(K, mp, plan, 2) > kLdsMax) --mp;
   if (M > 16 && mp <= 16) mp = 0;
-  // (what no chunk of the fused kernel serves stays refused below)
+  // (more chunks than a grid, or not a row in the LDS, stay refused below)
   const int mu = swiglu_rows_per_chunk(K, M);
   const int rows = mp > 0 ? mp : mu;
-  if (mu >= 1 && (M + mu - 1) / mu <= 65535 &&
+  if (rows >= 1 && (M + rows - 1) / rows <= 65535 &&
       swiglu_gemm_serves(P.n[0], K, M, (M + rows - 1) / rows))
     return launch_gemm_swiglu<PACKED>(P.w[0], P.s[0], P.w[1], P.s[1], X, P.y[0], P.n[0], K, M, stream);
   if (mp > 0) {

@@ -116,6 +116,14 @@ def test_bf16_gemv_more_row_chunks_than_a_grid(w4):
     assert w4.lib().cudalm_bf16_gemv_prepacked(fake, fake, fake, N, K, M, None) == w4.ERANGE
 
 
+def test_swiglu_more_row_chunks_than_a_grid(w4):
+    # K = 2048 leaves 25 rows per chunk of the kernel that serves N <= 4096
+    fake, N, K, M = 0x1000, 2048, 2048, 65535 * 25 + 1
+    for prepacked in (0, 1):
+        assert w4.lib().cudalm_w4a16_swiglu_bf16(fake, fake, fake, fake, fake, fake, N, K, M,
+                                                 prepacked, None) == w4.ERANGE
+
+
 def test_bf16_repack_preconditions_rejected_before_device(w4):
     # include/cudalm_bf16_gemv.h: the packed path needs N % 16 == 0,
     # K % 256 == 0 and 16-byte aligned bases
