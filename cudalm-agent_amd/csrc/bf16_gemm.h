@@ -8,7 +8,7 @@
 
 namespace cudalm_hip {
 
-// Whether the tile numbers fit the kernel's 32-bit indices.
+// Whether the tiles fit one launch.
 bool bf16_gemm_fits(int N, int M);
 
 template <bool PACKED>

@@ -210,7 +210,8 @@ int launch_gemm_t(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, int 
 }  // namespace
 
 bool bf16_gemm_fits(int N, int M) {
-  return static_cast<long long>((M + 63) / 64) * ((N + 127) / 128) < (1LL << 30);
+  const int bm = M <= 64 ? 64 : 128;
+  return static_cast<long long>((M + bm - 1) / bm) * ((N + 127) / 128) <= kMaxGemmTiles;
 }
 
 template <bool PACKED>

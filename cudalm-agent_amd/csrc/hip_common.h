@@ -19,6 +19,10 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
+// Workgroups of 256 threads in one launch whose grid is rounded up to a multiple
+// of 8: a launch numbers its threads in 32 bits.
+constexpr long long kMaxGemmTiles = (1LL << 24) - 8;
+
 constexpr size_t kLdsMax = 160 * 1024;  // LDS per CU (and per workgroup) on gfx950
 
 // Orders one wave's LDS writes before its later LDS reads (and those reads

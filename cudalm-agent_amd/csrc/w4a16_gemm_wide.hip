@@ -542,12 +542,14 @@ WideArgs wide_args(const uint8_t* W0, const uint16_t* S0, const uint8_t* W1, con
   return WideArgs{{W0, W1}, {S0, S1}, X, Y, N, K, M, 0, 0};
 }
 
-// Tiles of BM x BN outputs, -1 beyond the kernel's index ranges (32-bit tile
-// numbers and lane offsets; M as in the other prefill kernels' grids).
+// Tiles of BM x BN outputs, -1 beyond the kernel's index ranges (32-bit thread
+// numbers and lane offsets; M as in the other prefill kernels' grids). A y of
+// about 275 GB reaches the first past K = 1024, in tiles of 64 x 128; the unit
+// GEMM's two-dimensional grid holds it.
 long long wide_tiles(int N, int K, int M, int bm, int bn) {
   if (K > (1 << 20) || M > 65535 * 32) return -1;
   const long long t = static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  return t < (1LL << 30) ? t : -1;
+  return t <= kMaxGemmTiles ? t : -1;
 }
 
 // Where the wide kernel beats the smaller-tiled prefill kernels. Two lines, in
@@ -618,12 +620,12 @@ bool wide_group_serves(const PrefillGroup& P, int K, int M) {
   long long t = 0, wide = 0, cols8 = 0;
   for (int j = 0; j < P.count; ++j) {
     const int N = P.n[j], bn = wide_tile_cols(K);
-    if (wide_tiles(N, K, M, 64, 128) < 0) return false;
+    if (wide_tiles(N, K, M, 64, bn) < 0) return false;
     t += static_cast<long long>((M + 63) / 64) * ((N + 255) / 256);
     wide += static_cast<long long>((M + 63) / 64) * ((N + bn - 1) / bn);
     cols8 += N <= 64 && K > 4 * kGroup ? 6 : 8LL * ((N + 127) / 128);
   }
-  if (t >= (1LL << 28) || 32 * t < wide_fill<PACKED>(K) * cu_count()) return false;
+  if (wide > kMaxGemmTiles || 32 * t < wide_fill<PACKED>(K) * cu_count()) return false;
   return wide_rounds_pay(PACKED, K, wide, (M + 31) / 32 * cols8);
 }
 

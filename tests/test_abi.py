@@ -124,6 +124,23 @@ def test_swiglu_more_row_chunks_than_a_grid(w4):
                                                  prepacked, None) == w4.ERANGE
 
 
+@pytest.mark.parametrize("rule,N,K,M,fits", [
+    # (launched threads are numbered in 32 bits: 2^24 workgroups of 256 are too many)
+    ("11wide_servesILb1EEEbiii", 65536, 1152, 65535 * 32, False),  # 64 x 128 tiles
+    ("11wide_servesILb0EEEbiii", 1 << 23, 2048, 16385, False),
+    ("11wide_servesILb1EEEbiii", 65536, 1024, 65535 * 32, True),  # 64 x 256
+    ("11wide_servesILb1EEEbiii", 65536, 1152, 1 << 20, True),
+    ("16wide_swiglu_fitsEiii", 65536, 1024, 65535 * 32, False),
+    ("16wide_swiglu_fitsEiii", 65536, 1024, 1 << 20, True),
+    ("14bf16_gemm_fitsEii", (1 << 30) - 16, None, 129, False),
+    ("14bf16_gemm_fitsEii", 1 << 29, None, 129, True),
+    ("14bf16_gemm_fitsEii", 1 << 29, None, 64, True)])
+def test_gemm_tiles_fit_a_launch(w4, rule, N, K, M, fits):
+    fn = getattr(w4.lib(), "_ZN10cudalm_hip" + rule)
+    fn.restype = ctypes.c_bool
+    assert fn(*(v for v in (N, K, M) if v is not None)) is fits
+
+
 def test_bf16_repack_preconditions_rejected_before_device(w4):
     # include/cudalm_bf16_gemv.h: the packed path needs N % 16 == 0,
     # K % 256 == 0 and 16-byte aligned bases
