@@ -1998,8 +1998,10 @@ bool piece_direct(int ntiles, int K, int M) {
 
 // 17 <= M <= 32 at long K, where x leaves room for one workgroup per CU or does
 // not fit the LDS at all: the prefill kernels, which stage it by units, unless a
-// split kernel serves the call (a tile per CU at most) or the tiles are so
-// many that the streamed weights bound both. us, stream kernel (two 16-row
+// split kernel serves the call (a tile per CU at most) or the 64-row blocks of
+// the unit GEMM, counted per projection, take more than one round: there the
+// streamed weights bound both, and a group of (239, 8145, 7938) x 2560, 257 blocks
+// of 1021 tiles, M = 17 takes 12.2 / 18.4. us, stream kernel (two 16-row
 // passes where x does not fit) / prefill kernels, prepacked: 6144 x 2432 M = 17
 // 12.9 / 9.6, 16384 x 2432 M = 32 14.5 / 10.7, 60000 x 2432 M = 32 21.8 / 26.2,
 // 2048 x 2432 M = 32 (no room for the split) 13.9 / 9.7; not fitting: 6144 x
@@ -2008,12 +2010,12 @@ bool piece_direct(int ntiles, int K, int M) {
 // 16.8, 512 x 9216 M = 17 42.3 / 26.8, M = 32 68.3 / 27.0; of 2,000 random calls of N
 // <= 2048, K from 4096 to 10240, none is slower. The piece split keeps 4096 x 4096 M = 17 8.7 / 11.5, M = 32
 // 11.3 / 11.4.
-bool prefer_prefill(int ntiles, int K, int M, bool packed) {
+bool prefer_prefill(int ntiles, long long blocks, int K, int M, bool packed) {
   if (M <= 16 || M > 32) return false;
   if (!stream_fits(K, M, packed)) return !piece_direct(ntiles, K, M);
   if (K <= 2 * kUnit * kGroup) return false;
   if (ntiles <= cu_count()) return !split_fits(K, M, packed) && !piece_direct(ntiles, K, M);
-  return ntiles <= 4 * cu_count();
+  return blocks <= cu_count();
 }
 
 template <bool PACKED>
@@ -2021,7 +2023,7 @@ int dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_t* Y
              int M, int variant, hipStream_t stream) {
   if (variant == CUDALM_W4A16_VARIANT_AUTO) {
     const int ntiles = (N + kTileRows - 1) / kTileRows;
-    if (M > 32 || prefer_prefill(ntiles, K, M, PACKED)) {
+    if (M > 32 || prefer_prefill(ntiles, (N + 63) / 64, K, M, PACKED)) {
       variant = CUDALM_W4A16_VARIANT_PREFILL;
     } else if (stream_fits(K, M, PACKED) || piece_direct(ntiles, K, M)) {
       const ProjTable P = single_table(W, S, Y, N);
@@ -2069,7 +2071,7 @@ int f16_dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_
   // (mc < M <= 32: two or more launches of the stream kernels, 4096 x 3584 M = 32
   // 15.5 us against 10.9, 512 x 9216 M = 17 31.8 / 27.6)
   if (M <= 65535 * 32 && (M > 32 || (M > 16 && mc < M) ||
-                          prefer_prefill((N + kTileRows - 1) / kTileRows, K, M, PACKED)))
+                          prefer_prefill((N + kTileRows - 1) / kTileRows, (N + 63) / 64, K, M, PACKED)))
     return launch_prefill<ActF16, PACKED>(W, S, X, Y, N, K, M, stream);
   for (int m0 = 0; m0 < M; m0 += mc) {
     const int rows = M - m0 < mc ? M - m0 : mc;
@@ -2176,10 +2178,13 @@ int cudalm_w4a16_gemv_bf16_multi(const cudalm_w4a16_proj* projs, int count, cons
              (prepacked || aligned(projs[j].scale, 2));
   }
   if (prepacked && !vec_ok) return CUDALM_W4A16_EALIGN;
-  long long tiles = 0;
-  for (int j = 0; j < count; ++j) tiles += (projs[j].N + kTileRows - 1) / kTileRows;
+  long long tiles = 0, blocks = 0;
+  for (int j = 0; j < count; ++j) {
+    tiles += (projs[j].N + kTileRows - 1) / kTileRows;
+    blocks += (projs[j].N + 63) / 64;
+  }
   const bool prefill = vec_ok && tiles <= (1LL << 30) && M <= 65535 * 32 &&
-                       (M > 32 || prefer_prefill(static_cast<int>(tiles), K, M, prepacked));
+                       (M > 32 || prefer_prefill(static_cast<int>(tiles), blocks, K, M, prepacked));
   if (prefill && count > 1) {
     // the prefill kernels: one launch over the tiles of all projections
     PrefillGroup g = {};

@@ -54,7 +54,11 @@ def test_prefill_kernel(w4, dev, packed, N, K, M, kernel):
 @pytest.mark.parametrize("packed,Ns,K,M,kernel", [
     (False, (18, 23, 33), 1024, 11605, "gemm_unit"), (True, (28, 47), 1024, 8091, "gemm_unit"),
     (True, (6144, 2048, 16, 16), 1024, 1024, "gemm_wide"),
-    (False, (3584, 3584), 1024, 512, "gemm_wide")])
+    (False, (3584, 3584), 1024, 512, "gemm_wide"),
+    # 17 to 32 rows of long K: one 64-row block past a round, and a round
+    (True, (239, 8145, 7938), 2560, 17, "w4a16_stream"),
+    (False, (9926, 1951, 4454), 2432, 25, "w4a16_stream"),
+    (True, (256, 8128, 8000), 2560, 17, "gemm_unit")])
 def test_prefill_group_kernel(w4, dev, packed, Ns, K, M, kernel):
     pairs = [_weights(dev, N, K) for N in Ns]
     x = _x(dev, M, K)
