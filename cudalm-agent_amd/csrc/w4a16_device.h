@@ -315,7 +315,7 @@ int launch_wide_group(const PrefillGroup& P, int K, int M, hipStream_t stream);
 
 // SwiGLU front half of M > 32 rows on GEMM tiles, and where those beat the
 // `chunks` chunks of at most 32 rows that the fused kernels would run.
-bool swiglu_gemm_serves(int N, int K, int M, int chunks);
+bool swiglu_gemm_serves(int N, int K, int M, int chunks, bool packed);
 template <bool PACKED>
 int launch_gemm_swiglu(const uint8_t* Wg, const uint16_t* Sg, const uint8_t* Wu,
                        const uint16_t* Su, const uint16_t* X, uint16_t* Y, int N, int K, int M,

@@ -1049,8 +1049,11 @@ template int launch_prefill_group<false>(const PrefillGroup&, int, int, hipStrea
 // 6.7; K = 2048: 192 (1024, M = 96) 8.5 / 10.2, 256 (M = 128) 15.4 / 10.3; K =
 // 3584: 128 (1024, M = 64) 13.2 / 15.6, 192 (M = 96) 24.7 / 15.7. (At K <= 1024 the
 // line lies where hardly a shape loses, not where the gains begin: M = 64 gains
-// from fewer tiles than M = 40, and file layout 3784 x 640, M = 35, 474 tiles, 6.7 /
-// 7.5, still does not.)
+// from fewer tiles than M = 40.) A second chunk of at most 16 rows costs half, and
+// of the file layout, whose scales the GEMM loads one by one below K = 1024, the
+// chunks keep those while a row tile has a CU: K = 768, M = 33 to 48 6.2 to 6.7 /
+// 7.2, K = 640 6.1 to 6.6 / 7.0, K = 384 and 512 1 to 10 % (K = 256 level, K = 128
+// and 896 the other way by 6 and 25 %).
 //
 // Past K = 1024 a chunk's workgroups have a CU each, and while all of them fit
 // one round the chunks are the faster: 1024 x 1152, M = 109 file layout, 256
@@ -1059,10 +1062,11 @@ template int launch_prefill_group<false>(const PrefillGroup&, int, int, hipStrea
 // there are, follows from the LDS: 25 to 32 up to K = 2304, 17 at K = 4096.) Of 1,500
 // random shapes past K = 1024 three lose by 4 to 14 %, where the last chunk has
 // two to four rows.
-bool swiglu_gemm_serves(int N, int K, int M, int chunks) {
+bool swiglu_gemm_serves(int N, int K, int M, int chunks, bool packed) {
   if (M <= 32) return false;
   const long long cols = (N + 15) / 16, tiles = cols * ((M + 31) / 32);
   const long long cus = cu_count();
+  if (!packed && M <= 48 && cols <= cus && K > 2 * kGroup && K <= 6 * kGroup) return false;
   if (K <= kUnit * kGroup) return 2 * tiles >= 3 * cus;
   if (cols * chunks <= cus) return false;
   return K <= 2 * kUnit * kGroup ? tiles >= cus : 4 * tiles >= 3 * cus;

@@ -1893,7 +1893,7 @@ int launch_swiglu(const ProjTable& P, const uint16_t* X, int K, int M, hipStream
   const int mu = swiglu_rows_per_chunk(K, M);
   const int rows = mp > 0 ? mp : mu;
   if (rows >= 1 && (M + rows - 1) / rows <= 65535 &&
-      swiglu_gemm_serves(P.n[0], K, M, (M + rows - 1) / rows))
+      swiglu_gemm_serves(P.n[0], K, M, (M + rows - 1) / rows, PACKED))
     return launch_gemm_swiglu<PACKED>(P.w[0], P.s[0], P.w[1], P.s[1], X, P.y[0], P.n[0], K, M, stream);
   if (mp > 0) {
     const int mc = mp;

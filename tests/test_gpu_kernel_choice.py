@@ -73,6 +73,10 @@ def test_prefill_group_kernel(w4, dev, packed, Ns, K, M, kernel):
     # the chunks' workgroups fit one round
     (False, 1024, 1152, 109, "split_piece_pair"), (False, 306, 2304, 359, "w4a16_swiglu"),
     (True, 434, 2816, 221, "w4a16_swiglu"),
+    # the second chunk has at most 16 rows
+    (False, 3672, 768, 35, "split_piece_pair"), (False, 3784, 640, 48, "split_piece_pair"),
+    (False, 3672, 768, 49, "gemm_unit_swiglu"), (True, 3672, 768, 35, "gemm_unit_swiglu"),
+    (False, 4097, 768, 35, "gemm_unit_swiglu"), (False, 3672, 896, 35, "gemm_unit_swiglu"),
     # they take two
     (True, 1112, 2560, 102, "gemm_unit_swiglu"), (False, 1024, 1152, 130, "gemm_unit_swiglu"),
     (True, 3584, 1024, 64, "gemm_unit_swiglu"), (True, 3584, 1024, 1000, "gemm_wide")])

@@ -107,7 +107,7 @@ def test_wide_equals_decode_kernels(w4, dev, N, K, M, wide, f16):
     # unit GEMM: 128- and 64-row tiles, two k-slices, more units than the slices
     # keep, ragged N
     (3584, 1024, 100, "gemm_unit_swiglu"), (8200, 384, 70, "gemm_unit_swiglu"),
-    (3101, 512, 40, "gemm_unit_swiglu"), (6001, 640, 33, "gemm_unit_swiglu"),
+    (4201, 512, 40, "gemm_unit_swiglu"), (6001, 640, 33, "gemm_unit_swiglu"),
     (1030, 3584, 97, "gemm_unit_swiglu"), (1024, 2048, 129, "gemm_unit_swiglu"),
     (1029, 9216, 100, "gemm_unit_swiglu"),
     # a few tiles short of it: the chunks
