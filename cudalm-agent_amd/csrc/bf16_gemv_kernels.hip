@@ -280,27 +280,36 @@ int launch_stream_ct(const uint16_t* W, const uint16_t* X, uint16_t* Y, int N, i
 // 256 CUs: K = 1024: 256 (8192, M = 64) 10.1 / 10.6, 512 (16384, M = 64) 11.9 /
 // 11.1, (4096, M = 256) 11.7 / 14.0, 1024 (8192, M = 256) 22.9 / 15.0; K = 512:
 // 512 7.2 / 7.0, 1024 11.9 / 9.4; tile-major copy, K = 1024: 512 (16384, M =
-// 64) 9.9 / 11.3, 768 (M = 96) 18.1 / 14.9; K = 3072 (24-row chunks, one workgroup per
-// CU): 176 (1024, M = 256) 22.6 / 34.7, 384 (8192, M = 64) 39.4 / 26.3.
+// 64) 9.9 / 11.3, 768 (M = 96) 18.1 / 14.9, K = 256 (chunks of 17 KB, several to a
+// CU) 768 (8176, M = 174) 4.7 / 6.5, 1024 to 1280 8.8 / 6.8; K = 3072 (24-row chunks,
+// one workgroup per CU): 176 (1024, M = 256) 22.6 / 34.7, 384 (8192, M = 64) 39.4 / 26.3.
 //
 // Past K = 1024 the chunks' time steps by rounds of one workgroup per CU; a
 // short last chunk costs less than a round, and counts by its rows at M > 64 of
 // the tile-major copy (4160 x 2304, M = 101, 260 workgroups, 22.5 / 28.6; 864 x
-// 3840, M = 362, 266, 34.5 / 45.2). The GEMM takes 11 us per 1024 k while its tiles
+// 3840, M = 362, 266, 34.5 / 45.2) and of the file layout past K = 4096 (628 x 7568, M =
+// 252 1.16 times). The GEMM takes 11 us per 1024 k while its tiles
 // fit one round, a round of chunks of the few rows that the LDS holds at long K
 // about half of that, so at M > 64 the chunks' second round still ties with it at
-// K = 4096, and is the faster one past that for the tile-major copy (3072 x 4352,
-// M = 111, 336, 44.2 / 51.0; 2016 x 5632, M = 108, 288, 46.3 / 64.7; 1280 x 7680, M =
-// 131, 280, 62.2 / 86.7) and past K = 8192 for the file layout, whose chunks load
-// slower (1152 x 8640, M = 158, 360, 79.0 / 96.4; below it 5 to 20 % either way, e.g.
-// 1511 x 7288, M = 180, 73.9 / 83.3, 425 x 6928, M = 423, 87.5 / 79.5).
+// K = 4096 (past K = 3072 up to a quarter of it wins: 1024 x 3840, M = 330, 272, 35.0 /
+// 44.5; 2288 x 3584, M = 154, 33.1 / 41.9), and is the faster one past that where rows
+// are whole 128-byte lines: the tile-major copy (3072 x 4352, M = 111, 336, 44.2 /
+// 51.0; 1280 x 7680, M = 131, 280, 62.2 / 86.7) and the file layout of K a multiple of
+// 64 (2019 x 6848, M = 113, 352, 60.8 / 76.9; median of 68 shapes 3 %). Other file
+// layouts load slower, and the chunks' second round pays past K = 8192 (1152 x
+// 8640, M = 158, 360, 79.0 / 96.4; K = 5000 to 8000 up to 25 % either way, median 8 % for
+// the GEMM).
 bool prefer_gemm(int N, int K, int M, int mc, bool packed) {
   if (M <= 32 || !bf16_gemm_fits(N, M)) return false;
   const long long cols = (N + 63) / 64, wgs = cols * ((M + mc - 1) / mc);
   const long long cus = cu_count();
-  if (K <= 1024) return wgs >= (M <= 64 && !packed ? 2 : 3) * cus;
-  if (M > 64 && K > (packed ? 4096 : 8192)) return wgs > 2 * cus;
-  if (M > 64 && packed && cols * M <= cus * mc) return false;
+  if (K <= 1024)
+    return wgs >= (M <= 64 ? (packed ? 3 : 2) : packed && K <= 256 ? 4 : 3) * cus;
+  if (M > 64) {
+    if (K > (packed || K % 64 == 0 ? 4096 : 8192)) return wgs > 2 * cus;
+    if (packed && K > 3072) return 4 * cols * M > 5 * cus * mc;
+    if (packed || K > 4096) return cols * M > cus * mc;
+  }
   return wgs > cus;
 }
 

@@ -94,6 +94,11 @@ def test_swiglu_kernel(w4, dev, packed, N, K, M, kernel):
     (True, 4160, 2304, 101, "gemv_stream"), (True, 864, 3840, 362, "gemv_stream"),
     (True, 3072, 4352, 111, "gemv_stream"), (True, 2016, 5632, 108, "gemv_stream"),
     (True, 1280, 7680, 131, "gemv_stream"), (False, 1152, 8640, 158, "gemv_stream"),
+    (True, 1024, 3840, 330, "gemv_stream"), (False, 2019, 6848, 113, "gemv_stream"),
+    (False, 628, 7568, 252, "gemv_stream"), (True, 8176, 256, 174, "gemv_stream"),
+    # a little more of them
+    (True, 2048, 3840, 330, "bf16_gemm"), (False, 2019, 6856, 180, "bf16_gemm"),
+    (False, 4200, 6848, 113, "bf16_gemm"), (True, 16384, 256, 174, "bf16_gemm"),
     # enough of them, and 64-row tiles
     (True, 2800, 2304, 192, "bf16_gemm"), (True, 8192, 5632, 108, "bf16_gemm"),
     (False, 8192, 3072, 64, "bf16_gemm"), (True, 8704, 2304, 64, "bf16_gemm"),
