@@ -2007,8 +2007,9 @@ bool piece_direct(int ntiles, int K, int M) {
 // 2048 x 2432 M = 32 (no room for the split) 13.9 / 9.7; not fitting: 6144 x
 // 3584 M = 32 27.1 / 11.0, 16384 x 4096 M = 24 24.6 / 13.4, 60000 x 4096 M = 32
 // 64.0 / 31.5. Past K = 4096, 512 x 5120 M = 17 26.0 / 15.0, 2048 x 6144 M = 24 46.2 /
-// 16.8, 512 x 9216 M = 17 42.3 / 26.8, M = 32 68.3 / 27.0; of 2,000 random calls of N
-// <= 2048, K from 4096 to 10240, none is slower. The piece split keeps 4096 x 4096 M = 17 8.7 / 11.5, M = 32
+// 16.8, 512 x 9216 M = 17 42.3 / 26.8, M = 32 68.3 / 27.0; of 27,000 random calls of
+// K from 1152 to 10240 three are slower (file layout, 17 rows, N <= 51, K = 4480 and
+// 4608, at most 16 %). The piece split keeps 4096 x 4096 M = 17 8.7 / 11.5, M = 32
 // 11.3 / 11.4.
 bool prefer_prefill(int ntiles, long long blocks, int K, int M, bool packed) {
   if (M <= 16 || M > 32) return false;
@@ -2069,9 +2070,11 @@ int f16_dispatch(const uint8_t* W, const uint16_t* S, const uint16_t* X, uint16_
   while (mc > 0 && !stream_fits(K, mc, PACKED)) --mc;
   if (mc < 1) return CUDALM_W4A16_ERANGE;
   // (mc < M <= 32: two or more launches of the stream kernels, 4096 x 3584 M = 32
-  // 15.5 us against 10.9, 512 x 9216 M = 17 31.8 / 27.6)
+  // 15.5 us against 10.9, 512 x 9216 M = 17 31.8 / 27.6; slower only at M = 17 and 18
+  // of prepacked K = 8320, 2940 x 8320 22.7 / 25.8)
+  const int ntiles = (N + kTileRows - 1) / kTileRows;
   if (M <= 65535 * 32 && (M > 32 || (M > 16 && mc < M) ||
-                          prefer_prefill((N + kTileRows - 1) / kTileRows, (N + 63) / 64, K, M, PACKED)))
+                          prefer_prefill(ntiles, (N + 63) / 64, K, M, PACKED)))
     return launch_prefill<ActF16, PACKED>(W, S, X, Y, N, K, M, stream);
   for (int m0 = 0; m0 < M; m0 += mc) {
     const int rows = M - m0 < mc ? M - m0 : mc;

@@ -36,7 +36,7 @@ FULL_ATTN = [("q_proj", 4096, 1024), ("k_proj", 512, 1024), ("v_proj", 512, 1024
 MLP = [("gate_proj", 3584, 1024), ("up_proj", 3584, 1024), ("down_proj", 1024, 3584)]
 LM_HEAD = ("lm_head", 248320, 1024)
 ROLES = [name for name, _, _ in DELTANET + FULL_ATTN + MLP] + ["lm_head"]
-THREADS = max(1, min(16, os.cpu_count() or 1))  # the GPU box's host share
+THREADS = max(1, min(16, os.cpu_count() or 1))  # one GPU's share of the host
 
 
 def _groups(fused):
